@@ -29,58 +29,10 @@
 
 #include "kernels.hpp"
 #include "krylov.hpp"
+#include "krylov_dev.hpp"
+#include "resident.hpp"
 
 namespace mtl4g {
-
-enum { PCM_NONE = 0, PCM_DIAG = 1, PCM_GENERAL = 2 };
-
-// basic_iteration::finished(Real) (basic_iteration.hpp:60-65,85-93,43-48)
-// followed by ++iter when the loop goes on.  NaN/Inf residuals stop the
-// solve with MTL4G_ERR_NONFINITE instead of running to max_iter.
-// finished() alone (no ++iter): sets done when the loop must stop
-__device__ __forceinline__ void iter_check(Ctl* c, double resid, double* hist) {
-    if (c->hist_n < c->hist_cap) hist[c->hist_n] = resid;
-    c->hist_n++;
-    c->resid = resid;
-    const bool conv = c->norm_r0 == 0 ? (resid <= c->atol)
-                                      : (resid <= c->rtol * c->norm_r0 || resid <= c->atol);
-    if (conv) { c->done = 1; return; }
-    if (c->i >= c->max_iter) { c->error = 1; c->done = 1; return; }
-    if (!isfinite(resid)) { c->status = MTL4G_ERR_NONFINITE; c->done = 1; return; }
-}
-
-__device__ __forceinline__ void iter_finished(Ctl* c, double resid, double* hist) {
-    iter_check(c, resid, hist);
-    if (c->done) return;
-    c->i++;
-    c->first = c->i <= 1;
-}
-
-__device__ __forceinline__ bool conv_test(const Ctl* c, double resid) {
-    return c->norm_r0 == 0 ? (resid <= c->atol) : (resid <= c->rtol * c->norm_r0 || resid <= c->atol);
-}
-
-// A recurrence residual this far above the last FP64 residual is refreshed
-// at once instead of iterating on.
-constexpr double kGrowth = 10.0;
-// Mixed-precision BiCGSTAB refreshes when its residual fell by this factor.
-constexpr double kBicgDelta = 1e-5;
-
-// Mixed precision, loop head on the recurrence residual: it only estimates
-// convergence, so an estimated stop (or the iteration limit) pauses the
-// recurrence and asks for an FP64 refresh, which decides.  A non-finite
-// residual also pauses it and discards the low-precision correction; a
-// residual that has grown by kGrowth since the last refresh is refreshed
-// before the recurrence goes on.
-__device__ __forceinline__ void mixed_check(Ctl* c, double resid32) {
-    if (!isfinite(resid32)) { c->want_ru = 1; c->pause = 1; c->drop = 1; return; }
-    if (conv_test(c, resid32)) { c->want_ru = 1; c->pause = 1; return; }
-    if (c->i >= c->max_iter) { c->want_ru = 1; c->pause = 1; c->limit = 1; return; }
-    if (resid32 > kGrowth * c->rmax) { c->want_ru = 1; c->pause = 1; return; }
-    c->i++;
-    c->first = c->i <= 1;
-    if (resid32 <= c->delta * c->rmax) c->want_ru = 1;
-}
 
 constexpr int32_t kMaxStall = 8;
 
@@ -233,6 +185,20 @@ struct EpiCgQ {
         c->alpha = (double)(static_cast<VT>(c->rho) / tot[0]);
         c->rho_1 = c->rho;
     }
+};
+
+// q = A*p alone (product timing beside iterations that run on the chip)
+template <typename VT>
+struct EpiCgTimed {
+    static constexpr int NP = 0;
+    struct Pre {};
+    VT* q;
+    Ctl* c;
+    __device__ bool skip() const { return false; }
+    __device__ void prepare() {}
+    __device__ Pre preload(int) const { return Pre{}; }
+    __device__ void operator()(int row, VT s, const Pre&, VT*) const { __builtin_nontemporal_store(s, q + row); }
+    __device__ void finish(const VT*) const {}
 };
 
 // x += alpha*p; (lazy(r) -= alpha*q) || (lazy(rr)= lazy_unary_dot(r)); then
@@ -1911,6 +1877,26 @@ static int run_typed(const mtl4g_matrix_s* A, const MT* val, const mtl4g_pc_s* P
     } else {
         M4_TRY((cg_init<VT, MT, VT, PCM_GENERAL>(A, val, d, W, x, b, s)));
     }
+    if (method == MTL4G_CG && pcm != PCM_GENERAL) {
+        const bool f64 = P && P->fmt == MTL4G_F64;
+        const void* dv = pcm != PCM_DIAG ? nullptr : f64 ? (const void*)P->inv_diag64.p : (const void*)P->inv_diag32.p;
+        const int vfmt = sizeof(MT) == 8 ? MTL4G_F64 : sizeof(MT) == 4 ? MTL4G_F32 : MTL4G_BF16;
+        // product timing: an iteration on the chip has no launch of its own for
+        // q = A*p, so one iteration runs per launch and the product's kernel is
+        // timed beside it on the same p (q is not read)
+        const bool timed = sizeof(VT) == 8 && g_timer.on;
+        auto product = [&]() -> int {
+            if (!timed) return MTL4G_OK;
+            timer_mark(s, true);
+            M4_TRY(launch_csr<VT>(A, val, W.vecs.p, EpiCgTimed<VT>{W.vecs.p + A->n, W.ctl.p}, (VT*)nullptr, nullptr, s));
+            timer_mark(s, false);
+            return MTL4G_OK;
+        };
+        bool ran = false;
+        M4_TRY(resident_cg<VT>(A, vfmt, dv, f64 ? MTL4G_F64 : MTL4G_F32, W, x, s, timed ? 1 : kResidentSteps, product,
+                               &ran));
+        if (ran) return MTL4G_OK;
+    }
     // Enqueue chunks of iterations and poll the stop flag between chunks.
     int32_t launched = 0, chunk = 2;
     for (;;) {
@@ -1988,7 +1974,8 @@ int krylov_run(const mtl4g_matrix_s* A, const mtl4g_pc_s* P, int method, int fmt
     }
     if (c.status != 0) {
         set_error(c.status == MTL4G_ERR_BREAKDOWN ? "unexpected orthogonality (breakdown)"
-                                                   : "non-finite residual");
+                  : c.status == MTL4G_ERR_TIMEOUT ? "a bounded wait between workgroups expired"
+                                                  : "non-finite residual");
         return c.status;
     }
     return c.error;
@@ -2560,6 +2547,12 @@ static int mixed_typed(mtl4g_matrix_s* A, const MT* val32, const mtl4g_pc_s* P, 
         return cg_iteration<float, MT, float, PCM_GENERAL>(A, val32, P, d, W, x32, s);
     };
     M4_TRY(refresh());   // initial FP64 residual (Ctl::init set)
+    if (pcm != PCM_GENERAL) {
+        bool ran = false;
+        M4_TRY(resident_cg<float>(A, sizeof(MT) == 4 ? MTL4G_F32 : MTL4G_BF16, d, MTL4G_F32, W, x32, s, kResidentSteps,
+                                  refresh, &ran));
+        if (ran) return MTL4G_OK;
+    }
     int32_t launched = 0, chunk = 2;
     for (;;) {
         M4_HIP(hipMemcpyAsync(W.h_ctl, W.ctl.p, sizeof(Ctl), hipMemcpyDeviceToHost, s));
@@ -2673,7 +2666,8 @@ int mixed_run(mtl4g_matrix_s* A, const mtl4g_pc_s* P, int method, int fmt, doubl
     if (refreshes) *refreshes = c.ru_count;
     if (c.status != 0) {
         set_error(c.status == MTL4G_ERR_BREAKDOWN ? "unexpected orthogonality (breakdown)"
-                                                   : "non-finite residual");
+                  : c.status == MTL4G_ERR_TIMEOUT ? "a bounded wait between workgroups expired"
+                                                  : "non-finite residual");
         return c.status;
     }
     return c.error;

@@ -22,6 +22,7 @@ struct Ctl {
     int32_t mixed, pause, want_ru, ru_count, limit, init, restart;
     int32_t stall;           // consecutive FP64 refreshes that did not halve the residual
     int32_t drop;            // the FP32 recurrence went non-finite: discard its correction
+    int32_t refused;         // resident launches in a row that did not get onto the chip
     unsigned ticket[4];
 };
 
@@ -38,6 +39,9 @@ struct Workspace {
     DevBuf<double> terms;     // 3n, reductions in MTL4's order (FP64 only)
     DevBuf<double> small;     // bicgstab_ell: tau, gamma, gamma_a, gamma_aa
     DevBuf<double> pc64;      // float vectors with ilu_0/ic_0: the sweeps' FP64 chains (2n)
+    DevBuf<double> rslots;    // resident CG: all-reduce slots and wait words (resident.hip)
+    DevBuf<unsigned> rwords;
+    bool shared_gpu = false;  // other solves run beside this one: no grid that must hold the whole GPU
     Ctl* h_ctl = nullptr;     // pinned mirror for polling
     ~Workspace() {
         if (h_ctl) (void)hipHostFree(h_ctl);

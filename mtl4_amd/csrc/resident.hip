@@ -1,0 +1,893 @@
+// resident.hip -- itl::cg + pc::identity / pc::diagonal (cg.hpp:38-111) with
+// the whole state of the recurrence on the chip.
+//
+// The three-launch iteration of krylov.hip pays a launch, a grid ramp and a
+// last-workgroup reduction per kernel: 21.7 us per iteration on a 64 x 64
+// Laplacian whose arithmetic takes none of it.  Here one launch runs up to
+// kResidentSteps iterations: a lane keeps its rows of x, r, p, z, the inverse
+// diagonal and its part of the matrix in registers, and the only traffic
+// between workgroups is the direction p (written once per iteration, read
+// where the matrix reaches into another workgroup's rows) and two all-reduced
+// sums.  A system of up to kResBS * 8 rows is one workgroup and needs
+// neither.
+//
+// Element-wise results are those of the epilogues in krylov.hip bit for bit
+// (p, q, x, r; rows summed in column order); the sums are combined in another
+// fixed order, which depends only on the system, so a solve is deterministic.
+//
+// Workgroups wait for each other (Sync below), so all of them must be on the
+// chip at once.  A launch first meets at a rendezvous with a bounded wait:
+// when the grid does not get onto the chip (another kernel holds its CUs) the
+// launch gives up before it has changed anything and the host tries again.
+// After the rendezvous every workgroup is running and every later wait ends;
+// those waits are bounded too and raise an abort flag.
+//
+// Ordering: the inter-workgroup protocol of internal.hpp (agent-scope stores
+// and loads; wait_memory before the store that announces).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <condition_variable>
+#include <map>
+#include <mutex>
+
+#include "kernels.hpp"
+#include "krylov_dev.hpp"
+#include "resident.hpp"
+
+namespace mtl4g {
+
+constexpr int kResBS = 512;                  // 8 waves per workgroup, 256 registers per lane
+constexpr int kResMaxGrid = 256;             // one workgroup per CU
+constexpr int kResHalo = 1024;               // diagonals this close are read from LDS, others from memory
+constexpr unsigned kResMeet = 5 * 100000;    // rendezvous: 5 ms of the 100 MHz clock
+constexpr unsigned kResPolls = 1u << 22;     // polls of a later wait before it gives up
+
+// ------------------------------------------------------------------ waits between workgroups
+// Sums: three generations of slots, each holding a pending pattern until the
+// workgroup's sum of that generation is stored; a workgroup that has passed
+// generation g knows that all have passed g - 1 and resets its slots of it
+// (= generation g + 2's).  Up to kResFlat workgroups every one publishes to
+// eight copies of a slot row (one per blockIdx % 8, so 1/8 of the readers
+// poll the same lines) and sums the row itself; more meet in eight groups
+// first.  Measured per all-reduce: 1.9 us (32 workgroups), 2.0 (64), 2.5
+// (128), 3.3 (256) flat; 2.6-2.8 in groups.
+constexpr int kResFlat = 128;
+constexpr uint64_t kResPending = 0x7ff5c3c3c3c3c3c3ull;   // signalling NaN: no sum ever is
+constexpr int kSlotRow = 2 * kResMaxGrid;                  // two sums per workgroup
+constexpr int kSlotGen = 8 * kSlotRow;                     // eight copies
+// words: rendezvous arrivals and state, abort flag (own 128-byte lines), then one p flag per workgroup
+enum { RW_ARRIVE = 0, RW_STATE = 32, RW_ABORT = 64, RW_FLAG = 96 };
+constexpr int kResWords = RW_FLAG + kResMaxGrid;
+
+__device__ __forceinline__ bool res_pending(double v) { return (uint64_t)__double_as_longlong(v) == kResPending; }
+
+struct ResSync {
+    double* slots;     // 3 * kSlotGen
+    unsigned* words;   // kResWords
+    int grid;
+};
+
+// Two neighbouring values polled until both are there; false when the wait
+// expired or another workgroup has given up.
+__device__ __forceinline__ bool res_poll2(const double* p, unsigned* abort, double& a, double& b) {
+    a = ld_agent(p);
+    b = ld_agent(p + 1);
+    unsigned it = 0;
+#pragma clang loop unroll(disable)
+    while (res_pending(a) || res_pending(b)) {
+        if ((++it & 255u) == 0 && ld_agent(abort) != 0u) return false;
+        if (it > kResPolls) {
+            st_agent(abort, 1u);
+            return false;
+        }
+        a = ld_agent(p);
+        b = ld_agent(p + 1);
+    }
+    return true;
+}
+
+// v of another lane of the wave by DPP, 0 where the row mask or the row's edge
+// leaves a lane without a source.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double res_dpp(double v) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, ROWS, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, ROWS, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float res_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, true));
+}
+__device__ __forceinline__ double res_lane(double v, int lane) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), lane);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ float res_lane(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+// lane 7 (15) of a row: sum of its lanes 0..7 (8..15)
+template <typename T>
+__device__ __forceinline__ T res_row8(T v) {
+    v += res_dpp<0x111, 0xf>(v);   // row_shr:1
+    v += res_dpp<0x112, 0xf>(v);   // row_shr:2
+    v += res_dpp<0x114, 0xf>(v);   // row_shr:4
+    return v;
+}
+// Sum over the wave, uniform, in a fixed order: shifts within rows of 16
+// lanes, then the row sums (six DPP steps instead of six trips through the
+// LDS crossbar: about 1 us less per iteration of a one-workgroup solve).
+template <typename T>
+__device__ __forceinline__ T res_wave(T v) {
+    v = res_row8(v);
+    v += res_dpp<0x118, 0xf>(v);   // row_shr:8
+    v += res_dpp<0x142, 0xa>(v);   // row_bcast:15 into rows 1, 3
+    v += res_dpp<0x143, 0xc>(v);   // row_bcast:31 into rows 2, 3
+    return res_lane(v, 63);
+}
+
+// Sums of two values over the whole grid, in a fixed order, known to every
+// lane on return.  a, b: this lane's partial sums; sh: 4 * kResNW values, used
+// by turns (gen % 2), so no barrier is needed behind the last read.  Returns
+// false when a wait expired.
+constexpr int kResNW = kResBS / kWave;
+static_assert(kResNW == 8, "the waves' sums of both values fill one row of 16 lanes");
+template <typename VT>
+struct ResShared {
+    VT part[2][2 * kResNW];
+    VT tot[2][2];
+    int ok[2];
+};
+template <typename VT, bool ONE>
+__device__ __forceinline__ bool res_allsum(const ResSync& S, int gen, VT a, VT b, ResShared<VT>& sh, VT& ta, VT& tb) {
+    const int l = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave, h = gen & 1;
+    a = res_wave(a);
+    b = res_wave(b);
+    if (l == 0) {
+        sh.part[h][w] = a;
+        sh.part[h][kResNW + w] = b;
+    }
+    __syncthreads();
+    if constexpr (ONE) {
+        const VT v = res_row8(l < 2 * kResNW ? sh.part[h][l] : VT(0));
+        ta = res_lane(v, kResNW - 1);
+        tb = res_lane(v, 2 * kResNW - 1);
+        return true;
+    }
+    if (w == 0) {
+        const VT v = res_row8(l < 2 * kResNW ? sh.part[h][l] : VT(0));
+        a = res_lane(v, kResNW - 1);
+        b = res_lane(v, 2 * kResNW - 1);
+        bool ok = true;
+        const int g = blockIdx.x & 7, m = blockIdx.x >> 3;
+        double* now = S.slots + (size_t)(gen % 3) * kSlotGen;
+        double* old = S.slots + (size_t)((gen + 2) % 3) * kSlotGen;
+        unsigned* ab = S.words + RW_ABORT;
+        const double pend = __longlong_as_double((long long)kResPending);
+        if (S.grid <= kResFlat) {
+            if (l < 8) {
+                st_agent(now + l * kSlotRow + 2 * blockIdx.x, (double)a);
+                st_agent(now + l * kSlotRow + 2 * blockIdx.x + 1, (double)b);
+            }
+            a = b = VT(0);
+            const double* row = now + g * kSlotRow;
+#pragma clang loop unroll(disable)
+            for (int i = l; i < S.grid; i += kWave) {
+                double va = 0, vb = 0;
+                ok = res_poll2(row + 2 * i, ab, va, vb) && ok;
+                a += (VT)va;
+                b += (VT)vb;
+            }
+            a = res_wave(a);
+            b = res_wave(b);
+            if (l < 8) {
+                st_agent(old + l * kSlotRow + 2 * blockIdx.x, pend);
+                st_agent(old + l * kSlotRow + 2 * blockIdx.x + 1, pend);
+            }
+        } else {
+            // groups of the workgroups with equal blockIdx % 8; the first
+            // of a group sums it and publishes to one row per group
+            const int gs = (S.grid - g + 7) / 8;
+            double* grp = now + g * kSlotRow;             // 2 * gs slots, gs <= 32
+            double* top = now + g * kSlotRow + 128;       // this group's copy of the 8 group sums
+            if (l == 0) {
+                st_agent(grp + 2 * m, (double)a);
+                st_agent(grp + 2 * m + 1, (double)b);
+            }
+            if (m == 0) {
+                double va = 0, vb = 0;
+                if (l < gs) ok = res_poll2(grp + 2 * l, ab, va, vb);
+                a = res_wave((VT)va);
+                b = res_wave((VT)vb);
+                if (l < 8) {
+                    st_agent(now + l * kSlotRow + 128 + 2 * g, (double)a);
+                    st_agent(now + l * kSlotRow + 128 + 2 * g + 1, (double)b);
+                }
+            }
+            double va = 0, vb = 0;
+            if (l < 8) ok = res_poll2(top + 2 * l, ab, va, vb) && ok;
+            a = res_wave((VT)va);
+            b = res_wave((VT)vb);
+            if (l == 0) {
+                st_agent(old + g * kSlotRow + 2 * m, pend);
+                st_agent(old + g * kSlotRow + 2 * m + 1, pend);
+            }
+            if (m == 0 && l < 8) {
+                st_agent(old + l * kSlotRow + 128 + 2 * g, pend);
+                st_agent(old + l * kSlotRow + 128 + 2 * g + 1, pend);
+            }
+        }
+        ok = __all(ok);
+        if (l == 0) {
+            sh.tot[h][0] = a;
+            sh.tot[h][1] = b;
+            sh.ok[h] = ok;
+        }
+    }
+    __syncthreads();
+    // the same for every lane: kept in scalar registers, the branches on them scalar
+    ta = res_lane(sh.tot[h][0], 0);
+    tb = res_lane(sh.tot[h][1], 0);
+    return __builtin_amdgcn_readfirstlane(sh.ok[h]) != 0;
+}
+
+// Slots pending, words zero, before each launch.
+__global__ void k_resident_begin(ResSync S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 3 * kSlotGen) S.slots[i] = __longlong_as_double((long long)kResPending);
+    if (i < kResWords) S.words[i] = 0u;
+}
+
+// All workgroups are on the chip (true), or the launch gives up (false): one
+// answer for the whole grid, taken by whoever moves the state from 0.
+__device__ __forceinline__ bool res_meet(const ResSync& S, int* sh) {
+    if (threadIdx.x == 0) {
+        unsigned* st = S.words + RW_STATE;
+        const unsigned before =
+            __hip_atomic_fetch_add(S.words + RW_ARRIVE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned expect = 0u;
+        if (before + 1u == (unsigned)S.grid)
+            __hip_atomic_compare_exchange_strong(st, &expect, 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t t0 = wall_clock64();
+        unsigned v;
+        while ((v = ld_agent(st)) == 0u) {
+            if (wall_clock64() - t0 > kResMeet) {
+                expect = 0u;
+                __hip_atomic_compare_exchange_strong(st, &expect, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        *sh = v == 1u;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*sh) != 0;
+}
+
+// p of this workgroup is stored: tell the others, then wait for the
+// workgroups within `neigh` of this one (all of p they own is then readable
+// with agent-scope loads).  Every lane's stores are complete before the flag.
+__device__ __forceinline__ bool res_exchange(const ResSync& S, int lb, int neigh, unsigned step, int* sh) {
+    wait_memory();
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+        const int l = threadIdx.x;
+        if (l == 0) st_agent(S.words + RW_FLAG + lb, step);
+        const int lo = max(0, lb - neigh), hi = min(S.grid - 1, lb + neigh);
+        bool ok = true;
+        unsigned* ab = S.words + RW_ABORT;
+#pragma clang loop unroll(disable)
+        for (int i = lo + l; i <= hi; i += kWave) {
+            unsigned it = 0;
+#pragma clang loop unroll(disable)
+            while (ld_agent(S.words + RW_FLAG + i) < step) {
+                if ((++it & 255u) == 0 && ld_agent(ab) != 0u) { ok = false; break; }
+                if (it > kResPolls) {
+                    st_agent(ab, 1u);
+                    ok = false;
+                    break;
+                }
+            }
+        }
+        ok = __all(ok);
+        if (l == 0) *sh = ok;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*sh) != 0;
+}
+
+// ------------------------------------------------------------------ the matrix of a lane's rows
+// Lane t of workgroup lb holds rows lb*R*BS + k*BS + t, k < R.
+
+struct ResArgs {
+    int32_t n;
+    // diagonal operand: offsets ascending, values slice-major; map: stored diagonal of |offset| (symmetric copy)
+    const int32_t *doff, *dmap;
+    const void* val;
+    int ndiag, nstored, sym, fmt, halo;
+    // CSR operand
+    const int32_t *rowptr, *col;
+    // vectors
+    void *x, *r, *p;
+    const void* d;
+    int dfmt;   // MTL4G_F64 / MTL4G_F32; d null: identity
+    int neigh;
+    Ctl* c;
+    double* hist;
+    int32_t steps;
+    ResSync S;
+};
+
+template <typename VT>
+__device__ __forceinline__ VT res_value(const void* v, int fmt, int64_t i) {
+    if (fmt == MTL4G_F64) return static_cast<VT>(static_cast<const double*>(v)[i]);
+    if (fmt == MTL4G_F32) return static_cast<VT>(static_cast<const float*>(v)[i]);
+    return static_cast<VT>(bf16_to_f32(static_cast<const uint16_t*>(v)[i]));
+}
+__device__ __forceinline__ bool res_absent(const void* v, int fmt, int64_t i) {
+    if (fmt == MTL4G_F64) return dia_absent(static_cast<const double*>(v)[i]);
+    if (fmt == MTL4G_F32) return dia_absent(static_cast<const float*>(v)[i]);
+    return dia_absent(static_cast<const uint16_t*>(v)[i]);
+}
+
+// Element i of a vector of at most 2^29 elements, at agent scope: a 32-bit
+// offset on a uniform base (no 64-bit address per lane).
+template <typename VT>
+__device__ __forceinline__ VT res_ld(const VT* p, int i) {
+    return ld_agent(reinterpret_cast<const VT*>(reinterpret_cast<const char*>(p) + (unsigned)i * (unsigned)sizeof(VT)));
+}
+
+// Diagonals (at most ND, |offset| <= halo but for the first and the last):
+// values in registers, the workgroup's p with `halo` neighbours on both sides
+// in LDS, the first and last diagonal's p from memory when they lie further
+// out.  Slot ND-1 is always the last diagonal; slots without one are absent.
+template <typename VT, int ND_, int R_>
+struct OpDia {
+    static constexpr int R = R_, ND = ND_, kRegs = R_ * ND_;
+    static constexpr bool kOne = true;   // runs as one workgroup without p in memory
+    static constexpr int LDS = R * kResBS + 2 * kResHalo;
+    VT v[R][ND];
+    unsigned mask[R];
+    unsigned full;      // bit k: every entry of every lane's row k is present (wave-uniform)
+    int off[ND];        // uniform
+    bool flo, fhi;      // the first / last diagonal is read from memory
+    int halo;
+    template <typename Args>
+    __device__ __forceinline__ void load(const Args& a, int row0) {
+        halo = a.halo;
+        full = 0;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            const int di = d == ND - 1 ? a.ndiag - 1 : d;
+            const bool has = d == ND - 1 || d < a.ndiag - 1;
+            off[d] = has ? __builtin_amdgcn_readfirstlane(a.doff[di]) : 0;
+        }
+        flo = off[0] < -halo;
+        fhi = off[ND - 1] > halo;
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int row = row0 + k * kResBS + (int)threadIdx.x;
+            mask[k] = 0;
+#pragma unroll
+            for (int d = 0; d < ND; d++) {
+                v[k][d] = VT(0);
+                const int di = d == ND - 1 ? a.ndiag - 1 : d;
+                const bool has = d == ND - 1 || d < a.ndiag - 1;
+                if (has && row < a.n) {
+                    const int src = a.sym && off[d] < 0 ? row + off[d] : row;
+                    const int st = a.sym ? a.dmap[di] : di;
+                    if (src >= 0) {
+                        const int64_t i = ((int64_t)(src / kWave) * a.nstored + st) * kWave + src % kWave;
+                        if (!res_absent(a.val, a.fmt, i)) {
+                            v[k][d] = res_value<VT>(a.val, a.fmt, i);
+                            mask[k] |= 1u << d;
+                        }
+                    }
+                }
+            }
+            if (__all(mask[k] == (1u << ND) - 1u)) full |= 1u << k;
+        }
+        full = __builtin_amdgcn_readfirstlane(full);
+    }
+    // own p into LDS (a barrier follows before product())
+    __device__ __forceinline__ void put(VT* lds, int k, VT p) const {
+        lds[halo + k * kResBS + (int)threadIdx.x] = p;
+    }
+    template <bool ONE, typename Args>
+    __device__ __forceinline__ void product(const Args& a, int row0, VT* lds, VT (&q)[R]) const {
+        const VT* p = static_cast<const VT*>(a.p);
+        VT gl[R], gh[R], h[2 * kResHalo / kResBS];
+        // the lane index is made opaque, so that the addresses below are formed
+        // again in every iteration instead of living in registers across it
+        unsigned t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        const int last = a.n - 1;
+#pragma unroll
+        for (int k = 0; k < R; k++) gl[k] = gh[k] = VT(0);
+        if constexpr (!ONE) {
+            if (flo)
+#pragma unroll
+                for (int k = 0; k < R; k++) gl[k] = res_ld(p, min(max(row0 + k * kResBS + (int)t + off[0], 0), last));
+            if (fhi)
+#pragma unroll
+                for (int k = 0; k < R; k++) gh[k] = res_ld(p, min(row0 + k * kResBS + (int)t + off[ND - 1], last));
+#pragma unroll
+            for (int i = 0; i < 2 * kResHalo / kResBS; i++) {
+                const int j = (int)t + i * kResBS;   // 0..2*halo: below the rows, then above them
+                const int row = j < halo ? row0 - halo + j : row0 + R * kResBS + j - halo;
+                h[i] = VT(0);
+                if (j < 2 * halo && row >= 0 && row <= last) h[i] = res_ld(p, row);
+            }
+#pragma unroll
+            for (int i = 0; i < 2 * kResHalo / kResBS; i++) {
+                const int j = (int)t + i * kResBS;
+                if (j < 2 * halo) lds[j < halo ? j : R * kResBS + j] = h[i];
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const VT* own = lds + (halo + k * kResBS + (int)t);
+            VT g[ND];
+#pragma unroll
+            for (int d = 0; d < ND; d++) {
+                if (!ONE && d == 0) g[d] = flo ? gl[k] : own[flo ? 0 : off[d]];
+                else if (!ONE && d == ND - 1) g[d] = fhi ? gh[k] : own[fhi ? 0 : off[d]];
+                else g[d] = own[off[d]];
+            }
+            VT acc = VT(0);
+            unsigned mk = mask[k];   // opaque: no lane mask per entry kept across iterations
+            asm volatile("" : "+v"(mk));
+            if ((full >> k) & 1u) {
+#pragma unroll
+                for (int d = 0; d < ND; d++) acc += v[k][d] * g[d];
+            } else {
+#pragma unroll
+                for (int d = 0; d < ND; d++) {
+                    const VT with = acc + v[k][d] * g[d];
+                    acc = (mk >> d) & 1u ? with : acc;
+                }
+            }
+            q[k] = acc;
+            // two rows' neighbours in registers at a time
+            if (R > 2 && k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+};
+
+// Any pattern: the workgroup's entries spread over its lanes (at most E each,
+// values and columns in registers), products through LDS, a lane sums each of
+// its rows in column order.
+template <typename VT, int E_, int R_>
+struct OpCsr {
+    static constexpr int R = R_, E = E_, kRegs = 0;
+    static constexpr bool kOne = false;
+    static constexpr int LDS = E * kResBS;
+    VT v[E];
+    int c[E];
+    int ra[R], re[R];
+    int nz;
+    template <typename Args>
+    __device__ __forceinline__ void load(const Args& a, int row0) {
+        const int t = (int)threadIdx.x;
+        const int r1 = min(row0 + R * kResBS, a.n);
+        const int j0 = a.rowptr[min(row0, a.n)];
+        nz = a.rowptr[r1] - j0;
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int j = t + e * kResBS;
+            v[e] = VT(0);
+            c[e] = 0;
+            if (j < nz) {
+                v[e] = res_value<VT>(a.val, a.fmt, j0 + j);
+                c[e] = a.col[j0 + j];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            const int row = row0 + k * kResBS + t;
+            ra[k] = re[k] = 0;
+            if (row < a.n) {
+                ra[k] = a.rowptr[row] - j0;
+                re[k] = a.rowptr[row + 1] - j0;
+            }
+        }
+    }
+    __device__ __forceinline__ void put(VT*, int, VT) const {}
+    template <bool ONE, typename Args>
+    __device__ __forceinline__ void product(const Args& a, int row0, VT* lds, VT (&q)[R]) const {
+        const VT* p = static_cast<const VT*>(a.p);
+        const int t = (int)threadIdx.x;
+        VT g[E];
+#pragma unroll
+        for (int e = 0; e < E; e++) g[e] = t + e * kResBS < nz ? ld_agent(p + c[e]) : VT(0);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int j = t + e * kResBS;
+            if (j < nz) lds[j] = v[e] * g[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            VT s = VT(0);
+            for (int j = ra[k]; j < re[k]; j++) s += lds[j];
+            q[k] = s;
+        }
+    }
+};
+
+// ------------------------------------------------------------------ the loop head
+// The scalars of the recurrence and of basic_iteration, held by every lane (the
+// sums are the same for all of them).  Only workgroup 0 writes *c, after every
+// workgroup has passed the rendezvous and so has read it.
+template <typename VT>
+struct ResLoop {
+    VT rho, rho_1, beta, alpha, pq, rr, rz;
+    double norm_r0, atol, stop, grown, fell, resid;
+    int i, hist_n, max_iter, hist_cap, done, error, status, pause, want_ru, drop, limit;
+    bool first, mixed;
+    __device__ __forceinline__ void init(const Ctl* c) {
+        first = c->first != 0;
+        mixed = c->mixed != 0;
+        rho = static_cast<VT>(c->rho);
+        rho_1 = static_cast<VT>(c->rho_1);
+        beta = static_cast<VT>(c->beta);
+        alpha = pq = rr = rz = VT(0);
+        norm_r0 = c->norm_r0;
+        atol = c->atol;
+        // conv_test: resid <= rtol*norm_r0 || resid <= atol (norm_r0 == 0: atol alone)
+        stop = norm_r0 == 0 ? atol : fmax(c->rtol * norm_r0, atol);
+        grown = kGrowth * c->rmax;
+        fell = c->delta * c->rmax;
+        i = c->i;
+        hist_n = c->hist_n;
+        max_iter = c->max_iter;
+        hist_cap = c->hist_cap;
+        done = error = status = pause = want_ru = drop = limit = 0;
+        resid = 0.0;
+    }
+    // alpha = rho / p.q  (cg.hpp:105)
+    __device__ __forceinline__ void direction() {
+        alpha = rho / pq;
+        rho_1 = rho;
+    }
+    // iter_finished / mixed_check (krylov_dev.hpp) on rr and, when the loop
+    // goes on, the next rho and beta  (cg.hpp:94-101); true: leave the kernel
+    __device__ __forceinline__ bool head(double* hist) {
+        resid = (double)std::sqrt(std::fabs(rr));
+        const bool conv = resid <= stop, out = i >= max_iter, bad = !isfinite(resid);
+        if (!mixed) {
+            if (blockIdx.x == 0 && threadIdx.x == 0 && hist_n < hist_cap) hist[hist_n] = resid;
+            hist_n++;
+            done = conv || out || bad;
+            if (done && !conv) {
+                if (out) error = 1;
+                else status = MTL4G_ERR_NONFINITE;
+            }
+        } else {
+            pause = bad || conv || out || resid > grown;
+            want_ru = pause || resid <= fell;
+            drop = bad;
+            limit = !bad && !conv && out;
+        }
+        if (!done && !pause) {
+            i++;
+            first = i <= 1;
+            beta = rz / rho_1;
+            rho = rz;
+        }
+        return done || want_ru;
+    }
+    __device__ __forceinline__ void leave(Ctl* c, bool ok) const {
+        c->refused = 0;
+        if (!mixed) c->resid = resid;
+        c->rr = (double)rr;
+        c->alpha = (double)alpha;
+        c->alpha_1 = (double)pq;
+        c->rho_1 = (double)rho_1;
+        c->rho = (double)rho;
+        c->beta = (double)beta;
+        c->i = i;
+        c->first = first;
+        c->hist_n = hist_n;
+        c->done = done;
+        c->error = error;
+        c->status = status;
+        c->pause = pause;
+        c->want_ru = want_ru;
+        if (drop) c->drop = 1;
+        if (limit) c->limit = 1;
+        if (!ok) {   // a wait expired: the solve ends with an error
+            c->status = MTL4G_ERR_TIMEOUT;
+            c->done = 1;
+        }
+    }
+};
+
+// ------------------------------------------------------------------ the recurrence
+// What bounds it: latency.  Per iteration a grid pays one exchange of p (store,
+// flag, poll, read: about 2.5 us) and two all-reduces (2-2.8 us each); one
+// workgroup pays two block reductions, three divisions and square roots and
+// the LDS reads of its rows.  Measured per iteration (FP64, diagonal
+// preconditioner; before: three launches): 64^2 Laplacian 21.7 -> 2.8 us,
+// 61^3 diffusion 27 -> 9.3 us, 80^3 12.4 us, 100^3 18 us.
+// ONE: the grid is one workgroup and the operand reads p from LDS alone.
+template <typename VT, typename Op, bool ONE>
+__global__ __launch_bounds__(kResBS) void k_cg_resident(ResArgs a) {
+    constexpr int R = Op::R;
+    // eight FP64 rows of seven diagonals fill the registers: x and the inverse
+    // diagonal of those live in LDS, read and written by their own lane only
+    constexpr bool XD_LDS = Op::kRegs * sizeof(VT) > 400;
+    __shared__ VT xd[XD_LDS ? 2 * R * kResBS : 1];
+    __shared__ VT lds[Op::LDS];
+    __shared__ ResShared<VT> sh;
+    __shared__ int flag;
+    const int t = (int)threadIdx.x;
+    // the operand's rows: consecutive workgroups of one XCD hold consecutive rows
+    const int G = ONE ? 1 : a.S.grid;
+    int lb = ONE ? 0 : (int)blockIdx.x;
+    if (G % kXcd == 0) lb = xcd_logical_block(lb, G / kXcd);
+    const int row0 = lb * R * kResBS;
+    if (a.c->done || a.c->pause || a.c->want_ru) return;   // the whole grid reads the same state
+    ResLoop<VT> L;
+    L.init(a.c);
+    VT* xg = static_cast<VT*>(a.x);
+    VT* rg = static_cast<VT*>(a.r);
+    VT* pg = static_cast<VT*>(a.p);
+    Op op;
+    op.load(a, row0);
+    VT xr[XD_LDS ? 1 : R], dr[XD_LDS ? 1 : R], r[R], p[R], z[R];
+    auto x = [&](int k) -> VT& { return XD_LDS ? xd[k * kResBS + t] : xr[XD_LDS ? 0 : k]; };
+    auto d = [&](int k) -> VT& { return XD_LDS ? xd[(R + k) * kResBS + t] : dr[XD_LDS ? 0 : k]; };
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int row = row0 + k * kResBS + t;
+        VT xk = VT(0), dk = VT(1);
+        r[k] = p[k] = z[k] = VT(0);
+        if (row < a.n) {
+            xk = xg[row];
+            r[k] = rg[row];
+            p[k] = L.first ? VT(0) : pg[row];
+            if (a.d) dk = res_value<VT>(a.d, a.dfmt, row);
+            z[k] = dk * r[k];
+        }
+        x(k) = xk;
+        d(k) = dk;
+    }
+    if (!ONE && !res_meet(a.S, &flag)) {
+        if (blockIdx.x == 0 && t == 0) a.c->refused++;
+        return;
+    }
+    bool ok = true;
+    unsigned step = 0;
+    int gen = 0;
+    for (;;) {
+        // p = z  or  p = z + beta*p  (cg.hpp:98-101)
+        unsigned to = (unsigned)t;
+        asm volatile("" : "+v"(to));
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            p[k] = L.first ? z[k] : z[k] + L.beta * p[k];
+            op.put(lds, k, p[k]);
+            const int row = row0 + k * kResBS + (int)to;
+            if (!ONE && row < a.n) st_agent(pg + row, p[k]);
+        }
+        step++;
+        if constexpr (!ONE) {
+            ok = res_exchange(a.S, lb, a.neigh, step, &flag);
+            if (!ok) break;
+        } else {
+            __syncthreads();
+        }
+        // q = A*p, p.q; alpha  (cg.hpp:103-105)
+        VT q[R];
+        op.template product<ONE>(a, row0, lds, q);
+        VT s0 = VT(0), s1 = VT(0);
+#pragma unroll
+        for (int k = 0; k < R; k++) s0 += p[k] * q[k];
+        ok = res_allsum<VT, ONE>(a.S, gen++, s0, VT(0), sh, L.pq, s1);
+        if (!ok) break;
+        L.direction();
+        // x += alpha*p; r -= alpha*q; r.r, r.(d.*r)  (cg.hpp:106-108)
+        s0 = s1 = VT(0);
+#pragma unroll
+        for (int k = 0; k < R; k++) {
+            x(k) = x(k) + L.alpha * p[k];
+            r[k] = r[k] - L.alpha * q[k];
+            z[k] = d(k) * r[k];
+            s0 += r[k] * r[k];
+            s1 += r[k] * z[k];
+        }
+        ok = res_allsum<VT, ONE>(a.S, gen++, s0, s1, sh, L.rr, L.rz);
+        if (!ok) break;
+        if (L.head(a.hist) || (int)step >= a.steps) break;
+    }
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int row = row0 + k * kResBS + t;
+        if (row < a.n) {
+            xg[row] = x(k);
+            rg[row] = r[k];
+            pg[row] = p[k];
+        }
+    }
+    if (blockIdx.x == 0 && t == 0) L.leave(a.c, ok);
+}
+
+// ------------------------------------------------------------------ host
+namespace {
+struct Units {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::map<int, int> used;   // device -> CUs held by resident grids
+};
+Units& units() {
+    static Units u;
+    return u;
+}
+}  // namespace
+
+ResidentClaim::ResidentClaim(int dev, int n, int total) : device(dev), units(std::min(n, total)) {
+    if (!units) return;
+    Units& u = mtl4g::units();
+    std::unique_lock<std::mutex> lk(u.mu);
+    u.cv.wait(lk, [&] { return u.used[device] + units <= total; });
+    u.used[device] += units;
+}
+
+ResidentClaim::~ResidentClaim() {
+    if (!units) return;
+    Units& u = mtl4g::units();
+    {
+        std::lock_guard<std::mutex> lk(u.mu);
+        u.used[device] -= units;
+    }
+    u.cv.notify_all();
+}
+
+enum { ROP_NONE = 0, ROP_DIA5 = 1, ROP_DIA7 = 2, ROP_CSR8 = 3, ROP_CSR16 = 4, ROP_CSR24 = 5 };
+
+template <typename VT, typename Op>
+static int resident_go(const ResArgs& a, bool share, hipStream_t s) {
+    if constexpr (Op::kOne) {
+        if (!share) {
+            hipLaunchKernelGGL((k_cg_resident<VT, Op, true>), dim3(1), dim3(kResBS), 0, s, a);
+            M4_HIP(hipGetLastError());
+            return MTL4G_OK;
+        }
+    }
+    hipLaunchKernelGGL((k_cg_resident<VT, Op, false>), dim3(a.S.grid), dim3(kResBS), 0, s, a);
+    M4_HIP(hipGetLastError());
+    return MTL4G_OK;
+}
+
+ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes) {
+    ResidentPlan P;
+    if (A->n != A->m || A->n == 0 || reduction_order() == MTL4G_ORDER_MTL4) return P;
+    const int64_t n = A->n;
+    const int cus = std::min(A->cus, kResMaxGrid);
+    const bool sym = A->kernel == MTL4G_SPMV_DIA_SYM;
+    if (A->kernel == MTL4G_SPMV_DIA || sym) {
+        const std::vector<int32_t>& off = sym ? A->h_dsym_off : A->h_dia_off;
+        const int nd = (int)off.size();
+        if (nd >= 2 && nd <= 7) {
+            int inner = 0;
+            for (int d = 1; d + 1 < nd; d++) inner = std::max(inner, std::abs(off[d]));
+            int lo = std::abs(off[0]), hi = std::abs(off[nd - 1]);
+            if (inner <= kResHalo) {
+                // the fewest rows per lane whose workgroups fit the GPU; two at
+                // least (64,000 rows: 7.1 us per iteration on 63 workgroups,
+                // 7.5 on 125), and one workgroup where the system fits it
+                for (int rl = 1; rl <= (vt_bytes == 4 ? 4 : 3); rl++) {
+                    const int64_t rows = (int64_t)kResBS << rl;
+                    const int64_t g = (n + rows - 1) / rows;
+                    if (g > cus || (g > 1 && n <= kResBS * 8)) continue;
+                    P.op = nd <= 5 ? ROP_DIA5 : ROP_DIA7;
+                    P.rows_log2 = rl;
+                    P.grid = (int)g;
+                    int halo = inner;
+                    if (lo <= kResHalo) halo = std::max(halo, lo);
+                    if (hi <= kResHalo) halo = std::max(halo, hi);
+                    P.halo = halo;
+                    const int64_t reach = std::max(lo, hi);
+                    P.neigh = (int)std::min<int64_t>(g, (reach + rows - 1) / rows);
+                    P.share = g > 1 || reach > halo;
+                    return P;
+                }
+            }
+        }
+    }
+    // one lane adds a row's products one after the other: no long rows
+    if (A->max_row > 64) return P;
+    for (int rl = 0; rl <= 3; rl++) {
+        const int64_t rows = (int64_t)kResBS << rl;
+        const int64_t g = (n + rows - 1) / rows;
+        if (g > cus) continue;
+        int64_t most = 0;
+        for (int64_t b = 0; b < g; b++)
+            most = std::max<int64_t>(most, A->h_rowptr[std::min(n, (b + 1) * rows)] - A->h_rowptr[b * rows]);
+        const int64_t e = (most + kResBS - 1) / kResBS;
+        if (e > 24) return P;
+        P.op = e <= 8 ? ROP_CSR8 : e <= 16 ? ROP_CSR16 : ROP_CSR24;
+        P.rows_log2 = rl;
+        P.grid = (int)g;
+        P.neigh = (int)g;
+        P.share = true;
+        return P;
+    }
+    return P;
+}
+
+template <typename VT>
+int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, const void* inv_diag, int dfmt,
+                    Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s) {
+    if (!W.rslots.p) {
+        M4_TRY(W.rslots.alloc(3 * kSlotGen));
+        M4_TRY(W.rwords.alloc(kResWords));
+    }
+    ResArgs a{};
+    a.n = A->n;
+    const bool sym = A->kernel == MTL4G_SPMV_DIA_SYM;
+    if (plan.op == ROP_DIA5 || plan.op == ROP_DIA7) {
+        a.doff = sym ? A->dsym_off.p : A->dia_off.p;
+        a.dmap = sym ? A->dsym_map.p : nullptr;
+        a.ndiag = sym ? A->ndsym : A->ndiag;
+        a.nstored = sym ? A->nsym : A->ndiag;
+        a.sym = sym;
+        a.val = fmt == MTL4G_F64   ? (const void*)(sym ? A->dsym_val.p : A->dia_val.p)
+                : fmt == MTL4G_F32 ? (const void*)(sym ? A->dsym_val32.p : A->dia_val32.p)
+                                   : (const void*)(sym ? A->dsym_valbf.p : A->dia_valbf.p);
+    } else {
+        a.rowptr = A->rowptr.p;
+        a.col = A->col.p;
+        a.val = fmt == MTL4G_F64   ? (const void*)A->val.p
+                : fmt == MTL4G_F32 ? (const void*)A->val32.p
+                                   : (const void*)A->valbf.p;
+    }
+    a.fmt = fmt;
+    a.halo = plan.halo;
+    a.neigh = plan.neigh;
+    a.x = x;
+    a.p = W.vecs.p;
+    a.r = W.vecs.p + 2 * (size_t)A->n;
+    a.d = inv_diag;
+    a.dfmt = dfmt;
+    a.c = W.ctl.p;
+    a.hist = W.hist.p;
+    a.steps = steps;
+    a.S = ResSync{W.rslots.p, W.rwords.p, plan.grid};
+    if (plan.share) {
+        hipLaunchKernelGGL(k_resident_begin, dim3((3 * kSlotGen + 255) / 256), dim3(256), 0, s, a.S);
+        M4_HIP(hipGetLastError());
+    }
+#define M4_RES_ROWS(OP, NE)                                                                        \
+    if (plan.rows_log2 == 1) return resident_go<VT, OP<VT, NE, 2>>(a, plan.share, s);              \
+    if (plan.rows_log2 == 2) return resident_go<VT, OP<VT, NE, 4>>(a, plan.share, s);              \
+    if constexpr (sizeof(VT) == 4 && std::is_same<OP<VT, NE, 2>, OpDia<VT, NE, 2>>::value)         \
+        if (plan.rows_log2 == 4) return resident_go<VT, OpDia<VT, NE, 16>>(a, plan.share, s);      \
+    return resident_go<VT, OP<VT, NE, 8>>(a, plan.share, s)
+#define M4_RES_CSR(NE)                                                                             \
+    if (plan.rows_log2 == 0) return resident_go<VT, OpCsr<VT, NE, 1>>(a, plan.share, s);           \
+    M4_RES_ROWS(OpCsr, NE)
+    switch (plan.op) {
+    case ROP_DIA5: M4_RES_ROWS(OpDia, 5);
+    case ROP_DIA7: M4_RES_ROWS(OpDia, 7);
+    case ROP_CSR8: M4_RES_CSR(8);
+    case ROP_CSR16: M4_RES_CSR(16);
+    case ROP_CSR24: M4_RES_CSR(24);
+    }
+#undef M4_RES_CSR
+#undef M4_RES_ROWS
+    return MTL4G_ERR_INVALID;
+}
+
+template int resident_launch<double>(const ResidentPlan&, const mtl4g_matrix_s*, int, const void*, int,
+                                     Workspace<double>&, double*, int32_t, hipStream_t);
+template int resident_launch<float>(const ResidentPlan&, const mtl4g_matrix_s*, int, const void*, int,
+                                    Workspace<float>&, float*, int32_t, hipStream_t);
+
+}  // namespace mtl4g

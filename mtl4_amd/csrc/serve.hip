@@ -313,6 +313,7 @@ int mtl4g_server_run(mtl4g_server S_, int32_t nreq, const int32_t* mat, const in
         (void)hipSetDevice(B->device);
         Workspace<double> W64;
         Workspace<float> W32;
+        W64.shared_gpu = W32.shared_gpu = true;   // the workers and the batched launches share the GPU
         DevBuf<float> x32;
         DevBuf<GenItem> dg;
         if (dg.alloc(1)) {

@@ -1,0 +1,192 @@
+"""itl::cg with its state on the chip (resident.hip): one launch for many
+iterations on systems whose rows fit the registers of the GPU's compute units.
+Compared with the launch-per-kernel loop (which runs MTL4's summation order)
+after a few iterations, where only the order of the sums differs, and with the
+oracle at convergence."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def m():
+    import mtl4_amd
+    return mtl4_amd
+
+
+def _tridiag(n):
+    rp = np.concatenate([[0], np.cumsum([1 if n == 1 else 2 if i in (0, n - 1) else 3 for i in range(n)])])
+    ci, va = [], []
+    for i in range(n):
+        for j in (i - 1, i, i + 1):
+            if 0 <= j < n:
+                ci.append(j)
+                va.append(2.5 + 0.001 * (i % 7) if i == j else -1.0)
+    return rp.astype(np.int32), np.array(ci, np.int32), np.array(va)
+
+
+def _matrix(kind, size):
+    from mtl4_amd import generators as gen
+    if kind == "tridiag":
+        return _tridiag(size)
+    if kind == "grid2d":
+        return gen.laplacian_setup(*size)
+    if kind == "grid3d":
+        return gen.laplacian3d(*size)
+    if kind == "diffusion":
+        return gen.diffusion3d(size, seed=3)
+    return gen.random_spd(size, seed=4, nnz_per_row=size % 13 + 6)
+
+
+# edges: one workgroup (4096 rows) and the next size, waves and workgroups that
+# end inside a row block, neighbours at the LDS halo (1024) and just beyond it
+# in one workgroup and in several, 2/4/8 rows per lane, the register limits of
+# the unstructured operand (8, 16, 24 entries per lane), the largest grid
+CASES = [("tridiag", 1), ("tridiag", 2), ("tridiag", 65), ("tridiag", 513), ("tridiag", 4096), ("tridiag", 4097),
+         ("grid2d", (4, 1024)), ("grid2d", (3, 1025)), ("grid2d", (4, 1023)), ("grid2d", (9, 1024)),
+         ("grid2d", (9, 1025)), ("grid2d", (64, 64)), ("grid2d", (517, 523)), ("grid3d", (7, 5, 3)),
+         ("grid3d", (33, 32, 31)), ("grid3d", (101, 103, 97)), ("diffusion", 17), ("diffusion", 65),
+         ("random", 37), ("random", 700), ("random", 70003), ("random", 140010), ("random", 262150)]
+
+
+def _few(m, A, P, b, steps, general):
+    """x and the iteration state after `steps` iterations."""
+    x = m.dense_vector(A.num_rows())
+    it = m.basic_iteration(b, steps, 0.0)
+    with m.reduction_order(m.ORDER_MTL4 if general else m.ORDER_TREE):
+        m.cg(A, x, b, P, it)
+    return x.numpy(), it
+
+
+@pytest.mark.parametrize("pc", ["diagonal", "identity"])
+@pytest.mark.parametrize("kind,size", CASES)
+def test_resident_cg_matches_launch_per_kernel_loop(m, kind, size, pc):
+    rp, ci, va = _matrix(kind, size)
+    n = len(rp) - 1
+    print("resident cg", kind, size, n, pc, flush=True)
+    A = m.compressed2D(n, n, rp, ci, va)
+    P = m.pc.diagonal(A) if pc == "diagonal" else None
+    b = A * m.dense_vector(np.random.default_rng(5).uniform(-1, 1, n))
+    # rounding of the sums only: n terms of either order differ by a few
+    # 1e-16 relative, amplified by at most a few per iteration
+    steps = min(6, n)
+    xa, ia = _few(m, A, P, b, steps, False)
+    xb, ib = _few(m, A, P, b, steps, True)
+    assert ia.iterations() == ib.iterations() and ia.error_code() == ib.error_code()
+    assert np.linalg.norm(xa - xb) <= 1e-12 * np.linalg.norm(xb)
+    xc, _ = _few(m, A, P, b, steps, False)
+    assert np.array_equal(xa, xc)   # deterministic
+
+
+@pytest.mark.parametrize("layout", ["dia", "sym"])
+@pytest.mark.parametrize("kind,size", [("grid2d", (61, 64)), ("grid2d", (7, 1500)), ("diffusion", 33)])
+def test_resident_cg_layouts_and_oracle(m, kind, size, layout):
+    import orc
+    rp, ci, va = _matrix(kind, size)
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    if layout == "sym":
+        A.set_kernel(m._lib.SPMV_DIA_SYM, 4, 4)
+    O = orc.Matrix(rp, ci, va)
+    xt = np.random.default_rng(6).uniform(-1, 1, n)
+    b = orc.spmv(O, xt)
+    xo, st, ito, _ = orc.cg(O, b, orc.Preconditioner("diagonal", O), max_iter=5000, rtol=1e-10)
+    x, bd = m.dense_vector(n), m.dense_vector(b)
+    it = m.basic_iteration(bd, 5000, 1e-10)
+    assert m.cg(A, x, bd, m.pc.diagonal(A), it) == 0 and st == 0
+    assert abs(it.iterations() - ito.i) <= 2
+    assert np.linalg.norm(x.numpy() - xo) <= 1e-9 * np.linalg.norm(xo)
+
+
+def test_resident_cg_history_start_vector_and_limits(m):
+    rp, ci, va = _matrix("grid2d", (64, 64))
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    P = m.pc.diagonal(A)
+    rng = np.random.default_rng(7)
+    x0 = rng.uniform(-1, 1, n)
+    b = m.dense_vector(rng.uniform(-1, 1, n))
+    import io
+    out = io.StringIO()
+    it = m.cyclic_iteration(b, 400, 1e-10, 0.0, 1, out)
+    x = m.dense_vector(x0)
+    assert m.cg(A, x, b, P, it) == 0
+    # one residual per finished() call, the last one reported and converged
+    assert len(it.history) == it.iterations() + 1 and it.history[-1] == it.resid()
+    assert it.resid() <= 1e-10 * it.norm_r0()
+    it2 = m.basic_iteration(b, it.iterations() - 1, 1e-10)
+    x2 = m.dense_vector(x0)
+    assert m.cg(A, x2, b, P, it2) == 1 and it2.iterations() == it.iterations() - 1
+    # more iterations than one launch runs: the state goes on in the next one
+    big = m.compressed2D(*([len(_matrix("diffusion", 33)[0]) - 1] * 2), *_matrix("diffusion", 33))
+    bb = m.dense_vector(rng.uniform(-1, 1, 33 ** 3))
+    itb = m.basic_iteration(bb, 700, 0.0)
+    xb = m.dense_vector(33 ** 3)
+    m.cg(big, xb, bb, m.pc.diagonal(big), itb)
+    assert itb.iterations() == 700 and np.isfinite(xb.numpy()).all()
+
+
+def test_resident_cg_nonfinite(m):
+    rp, ci, va = _matrix("grid2d", (40, 40))
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    b = np.ones(n)
+    b[17] = np.inf
+    bd, x = m.dense_vector(b), m.dense_vector(n)
+    with pytest.raises(m.nonfinite_error):
+        m.cg(A, x, bd, m.pc.diagonal(A), m.basic_iteration(1.0, 50, 1e-10))
+
+
+def test_resident_cg_concurrent_threads(m):
+    """Solves of several threads on streams of their own: each gets the bits of
+    the same solve alone."""
+    import torch
+    jobs = []
+    for k, size in enumerate([(300, 301), (64, 64), (200, 333), (517, 523)]):
+        rp, ci, va = _matrix("grid2d", size)
+        n = len(rp) - 1
+        A = m.compressed2D(n, n, rp, ci, va)
+        b = m.dense_vector(np.random.default_rng(k).uniform(-1, 1, n))
+        P = m.pc.diagonal(A)
+        x = m.dense_vector(n)
+        m.cg(A, x, b, P, m.basic_iteration(b, 300, 1e-12))
+        jobs.append((A, b, P, n, x.numpy()))
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(job):
+        A, b, P, n, want = job
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(3):
+                x = m.dense_vector(n)
+                m.cg(A, x, b, P, m.basic_iteration(b, 300, 1e-12))
+                if not np.array_equal(x.numpy(), want):
+                    bad.append(n)
+
+    ts = [threading.Thread(target=work, args=(j,)) for j in jobs]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    assert not bad and not any(t.is_alive() for t in ts)
+
+
+# BF16 matrix values converge on the well-conditioned systems only
+@pytest.mark.parametrize("kind,size,fmt", [("random", 2000, "F32"), ("random", 2000, "BF16"),
+                                           ("grid2d", (40, 41), "F32"), ("diffusion", 20, "F32"),
+                                           ("random", 90000, "F32"), ("random", 90000, "BF16")])
+def test_resident_mixed_cg(m, kind, size, fmt):
+    rp, ci, va = _matrix(kind, size)
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    xt = np.random.default_rng(8).uniform(-1, 1, n)
+    b = A * m.dense_vector(xt)
+    x = m.dense_vector(n)
+    err, st = m.ir_solve(A, x, b, m.basic_iteration(b, 20000, 1e-10), m.pc.diagonal(A, m.F32),
+                         value_format=getattr(m, fmt))
+    assert err == 0 and st["relres"] <= 1e-10
+    r = b.numpy() - (A * x).numpy()
+    assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b.numpy())
