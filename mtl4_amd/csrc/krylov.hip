@@ -1691,10 +1691,9 @@ static int ensure_workspace(Workspace<VT>& W, int32_t n, int nvec, const mtl4g_p
     const bool sweeps = P && (P->kind == MTL4G_PC_ILU0 || P->kind == MTL4G_PC_IC0);
     if (sweeps && sizeof(VT) == 4 && W.pc64.n < 2 * (size_t)n) M4_TRY(W.pc64.alloc(2 * (size_t)std::max(n, 1)));
     size_t words = sweeps ? pc_counter_words(P) : 1;
-    if (W.pc_counters.n < words) {
-        M4_TRY(W.pc_counters.alloc(words));
-        M4_TRY(zero_on(W.pc_counters.p, words * sizeof(unsigned), s));
-    }
+    if (W.pc_counters.n < words) M4_TRY(W.pc_counters.alloc(words));
+    // zeroed for every solve: a sweep that gave up leaves them as they were
+    if (sweeps) M4_TRY(zero_on(W.pc_counters.p, W.pc_counters.n * sizeof(unsigned), s));
     return MTL4G_OK;
 }
 

@@ -330,9 +330,19 @@ static int build_chain(const SweepRows& R, int fmt, Sweep* S) {
     const int64_t T = (int64_t)C->Tx * C->Ty;
     C->stile = ((int64_t)Lc + C->Tx + C->Ty - 2) * T;
     C->nslots = C->stile * C->tiles_x * C->tiles_y;
+    C->xy = ndep >= 2 ? ((int64_t)Lc + C->Ty - 1) * C->Ty : 0;
+    C->xtile = C->xy + (ndep >= 3 ? ((int64_t)Lc + C->Tx - 1) * C->Tx : 0);
     // every byte offset the kernel forms stays below its out-of-range
     // marker 0x7ffffff0; else the level schedule stays
-    if ((C->nslots * ndep + 1024) * 8 >= 0x7ffffff0) return MTL4G_OK;
+    if ((C->nslots * ndep + 2 * kChainTail) * 8 >= 0x7ffffff0) return MTL4G_OK;
+    // entries every row inside the grid has: one per offset that stays in it
+    {
+        const int64_t rows_e0 = (int64_t)Cx * Cy, rows_x0 = (int64_t)Lc * Cy, rows_y0 = (int64_t)Lc * Cx;
+        int64_t full = n - rows_e0;
+        if (ndep >= 2) full += n - rows_x0;
+        if (ndep >= 3) full += n - rows_y0;
+        C->holes = (int64_t)R.rowptr[n] != full;
+    }
     const int64_t ns = C->nslots;
     auto slot = [&](int64_t d) { return d == 1 ? 0 : d == Lc ? 1 : 2; };
     const bool gathered = !R.dsrc.empty();
@@ -365,20 +375,20 @@ static int build_chain(const SweepRows& R, int fmt, Sweep* S) {
         M4_TRY(up(C->src, src));
         M4_TRY(up(C->dsrc, dsrc));
         if (fmt == MTL4G_F64) {
-            M4_TRY(C->val64.alloc(nv));
-            M4_TRY(C->dia64.alloc(ns));
+            M4_TRY(C->val64.alloc(nv + kChainTail));
+            M4_TRY(C->dia64.alloc(ns + kChainTail));
         } else if (fmt == MTL4G_F32) {
-            M4_TRY(C->val32.alloc(nv));
-            M4_TRY(C->dia32.alloc(ns));
+            M4_TRY(C->val32.alloc(nv + kChainTail));
+            M4_TRY(C->dia32.alloc(ns + kChainTail));
         } else {
-            M4_TRY(C->val16.alloc(nv));
-            M4_TRY(C->dia16.alloc(ns));
+            M4_TRY(C->val16.alloc(nv + kChainTail));
+            M4_TRY(C->dia16.alloc(ns + kChainTail));
         }
     } else {
         auto fill = [&](auto& vbuf, auto& dbuf, auto absent, auto conv) -> int {
             using T = decltype(absent);
-            std::vector<T> v(nv), dg(ns);
-            for (size_t i = 0; i < nv; i++) v[i] = present[i] ? conv(val[i]) : absent;
+            std::vector<T> v(nv + kChainTail, absent), dg(ns + kChainTail, conv(1.0));
+            for (size_t i = 0; i < nv; i++) v[i] = present[i] ? conv(val[i]) : C->holes ? absent : conv(0.0);
             for (int64_t i = 0; i < ns; i++) dg[i] = conv(dia[i]);
             M4_TRY(up(vbuf, v));
             return up(dbuf, dg);
@@ -402,13 +412,13 @@ int fill_chain(ChainSweep& C, int fmt, const double* fval, hipStream_t s) {
     const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((n * C.ndep + 1023) / 1024, 2048));
     const int32_t* dsrc = C.unit ? nullptr : C.dsrc.p;
     if (fmt == MTL4G_F64)
-        hipLaunchKernelGGL(k_fill_chain<double>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.src.p, dsrc, fval,
+        hipLaunchKernelGGL(k_fill_chain<double>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.holes, C.src.p, dsrc, fval,
                            C.val64.p, C.dia64.p);
     else if (fmt == MTL4G_F32)
-        hipLaunchKernelGGL(k_fill_chain<float>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.src.p, dsrc, fval,
+        hipLaunchKernelGGL(k_fill_chain<float>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.holes, C.src.p, dsrc, fval,
                            C.val32.p, C.dia32.p);
     else
-        hipLaunchKernelGGL(k_fill_chain<uint16_t>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.src.p, dsrc, fval,
+        hipLaunchKernelGGL(k_fill_chain<uint16_t>, dim3(grid), dim3(256), 0, s, n, C.ndep, C.holes, C.src.p, dsrc, fval,
                            C.val16.p, C.dia16.p);
     M4_HIP(hipGetLastError());
     return MTL4G_OK;
@@ -417,8 +427,9 @@ int fill_chain(ChainSweep& C, int fmt, const double* fval, hipStream_t s) {
 template <typename MT, typename IT, bool LOWER, bool UNIT>
 static void launch_chain_t(const ChainSweep& C, const MT* val, const MT* dia, const IT* v, double* w, float* w32,
                            unsigned* counters, int* err, const int* skip, hipStream_t s) {
-    ChainView<MT> V{val, dia, C.n, C.Lc, C.Cx, C.Cy, C.Tx, C.Ty, C.tiles_x, (int32_t)C.stile, (int32_t)C.nslots};
-    const dim3 grid(C.tiles_x * C.tiles_y), block(C.Tx * C.Ty);
+    ChainView<MT> V{val, dia, C.n, C.Lc, C.Cx, C.Cy, C.Tx, C.Ty, C.tiles_x, (int32_t)C.stile, (int32_t)C.nslots,
+                    C.holes ? 1 : 0, C.xtile, C.xy};
+    const dim3 grid(C.tiles_x * C.tiles_y), block(5 * kWave);
     if (C.ndep == 1)
         hipLaunchKernelGGL((k_chain<MT, IT, LOWER, UNIT, 1>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
     else if (C.ndep == 2)
@@ -542,8 +553,8 @@ int upload_sweep(const SweepRows& R, int fmt, Sweep* S) {
         M4_TRY(up(S->dia16, d16));
     }
     M4_TRY(build_chain(R, fmt, S));
-    M4_TRY(S->counters.alloc(sweep_counter_words(nlev)));
-    M4_HIP(hipMemset(S->counters.p, 0, sweep_counter_words(nlev) * sizeof(unsigned)));
+    M4_TRY(S->counters.alloc(S->words()));
+    M4_HIP(hipMemset(S->counters.p, 0, S->words() * sizeof(unsigned)));
     // complete before any stream (including non-blocking ones) uses the counters
     M4_HIP(hipDeviceSynchronize());
     return MTL4G_OK;
@@ -694,16 +705,21 @@ static int grid_for(int64_t n) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(g, 2048));
 }
 
+size_t Sweep::words() const {
+    if (!chain) return sweep_counter_words(nlev);
+    return chain_counter_words + 2 * (size_t)(chain->xtile * chain->tiles_x * chain->tiles_y);
+}
+
 template <typename IT, typename VT>
 int launch_sweep(const Sweep& S, int fmt, const IT* v, VT* w, float* w32, const int* skip, int* err,
                  unsigned* counters, hipStream_t s) {
     if (S.n == 0) return MTL4G_OK;
     if (!counters) counters = S.counters.p;
-    hipLaunchKernelGGL(k_fill_pending<VT>, dim3(grid_for(S.n)), dim3(256), 0, s, (int64_t)S.n, w, skip);
     if (S.chain) {
         static_assert(std::is_same<VT, double>::value, "the chain pipeline keeps its results in FP64");
         return launch_chain<IT>(*S.chain, fmt, v, w, w32, counters, err, skip, s);
     }
+    hipLaunchKernelGGL(k_fill_pending<VT>, dim3(grid_for(S.n)), dim3(256), 0, s, (int64_t)S.n, w, skip);
     if (fmt == MTL4G_F64) {
         SweepView<double, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
                                 S.blk_level.p, S.val64.p, S.dia64.p, S.nlev, S.unit ? 1 : 0};
@@ -731,7 +747,7 @@ template int launch_sweep<float, double>(const Sweep&, int, const float*, double
 
 
 size_t pc_counter_words(const mtl4g_pc_s* P) {
-    return sweep_counter_words(P->lower.nlev) + sweep_counter_words(P->upper.nlev);
+    return P->lower.words() + P->upper.words();
 }
 
 template <typename VT>
@@ -755,7 +771,7 @@ int pc_apply(const mtl4g_pc_s* P, const VT* r, VT* z, VT* y0, const int* skip,
                                P->inv_diag16.p, r, z, skip);
         break;
     default: {
-        unsigned* cu = counters ? counters + sweep_counter_words(P->lower.nlev) : nullptr;
+        unsigned* cu = counters ? counters + P->lower.words() : nullptr;
         if constexpr (sizeof(VT) == 8) {
             M4_TRY((launch_sweep<double, double>(P->lower, P->fmt, r, y0, nullptr, skip, P->err.p, counters, s)));
             M4_TRY((launch_sweep<double, double>(P->upper, P->fmt, y0, z, nullptr, skip, P->err.p, cu, s)));
@@ -790,7 +806,11 @@ int pc_check_error(const mtl4g_pc_s* P, hipStream_t s) {
     M4_HIP(hipMemcpyAsync(&h, P->err.p, sizeof(int), hipMemcpyDeviceToHost, s));
     M4_HIP(hipStreamSynchronize(s));
     if (h) {
+        // the handle's own counters and exchange slots are where the abandoned
+        // launch left them; a caller drops its own
         M4_HIP(hipMemsetAsync(P->err.p, 0, sizeof(int), s));
+        for (const Sweep* w : {&P->lower, &P->upper, &P->adj_lower, &P->adj_upper})
+            if (w->counters.p) M4_HIP(hipMemsetAsync(w->counters.p, 0, w->counters.n * sizeof(unsigned), s));
         set_error("triangular sweep: a bounded level wait expired");
         return MTL4G_ERR_TIMEOUT;
     }

@@ -37,6 +37,10 @@ struct Sweep {
     std::unique_ptr<ChainSweep> chain;   // grid-structured factor: the chain pipeline runs instead
     Sweep();
     ~Sweep();
+    // words of a caller's counters, zeroed before the first launch: the level
+    // schedule's (sweep_counter_words), or the chain pipeline's three counters
+    // and its exchange slots
+    size_t words() const;
 };
 
 // Host description of a sweep before upload: rows in natural order.
@@ -57,8 +61,8 @@ int upload_sweep(const SweepRows& rows, int value_format, Sweep* S);
 // (rounded to float for MTL4G_F32 storage)
 int fill_sweep(Sweep& S, int value_format, const double* fval, hipStream_t s);
 
-// counters: sweep_counter_words(nlev) zeroed words owned by the caller (NULL =
-// the sweep's own); each launch leaves them zeroed again.
+// counters: S.words() zeroed words owned by the caller (NULL = the sweep's
+// own); each launch leaves them zeroed again.
 // The row arithmetic runs in VT; v is read as IT; w32 (may be null) also
 // receives the results rounded to float.
 template <typename IT, typename VT>
