@@ -26,15 +26,17 @@
 #include "batched.hpp"
 #include "kernels.hpp"
 #include "precond.hpp"
+#include "wave_dpp.hpp"
 
 namespace mtl4g {
 
 enum { BPC_NONE = 0, BPC_DIAG = 1, BPC_ILU = 2 };
 
+// Sums of a and b over the workgroup, in a fixed order, in every thread.
 template <int BS, typename T>
 __device__ __forceinline__ void block_sum2(T& a, T& b, T* sh) {
-    a = wave_sum(a);
-    b = wave_sum(b);
+    a = res_wave(a);
+    b = res_wave(b);
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     __syncthreads();
     if (lane == 0) {
@@ -52,31 +54,97 @@ __device__ __forceinline__ void block_sum2(T& a, T& b, T* sh) {
     b = rb;
 }
 
-// one row of the product, column order (mat_vec_mult.hpp:656-682); the
-// indices and values of eight entries are requested together, then their
-// eight gathers, so a row costs two memory round trips per eight entries
-template <typename AT, typename MT, typename VT>
-__device__ __forceinline__ AT brow(const BatchDev& M, const MT* __restrict__ val, int grow, int r0,
-                                   const VT* __restrict__ v) {
-    AT s = 0;
-    const int j0 = M.rowptr[grow], j1 = M.rowptr[grow + 1];
-    for (int j = j0; j < j1; j += 8) {
-        int c[8];
-        AT m[8], g[8];
+// Rows (elements) a thread works on at once.  A row costs three dependent
+// memory round trips (bounds, entries, gathers) and a thread has n/BS of them
+// in turn, so a workgroup of 256 spent 130 us per iteration on 16,384 rows;
+// the trips of several rows overlap.  160 systems of up to 16,384 rows, FP64,
+// one row of two or four entries at a time against these: 256 threads 73.0 ->
+// 37.2 ms, 512 threads 39.1 -> 29.8, 1024 threads 31.4 -> 28.5 (one row of up
+// to eight entries: sixteen waves hide the rest, and with half the registers
+// two rows spill, 29.1).
+template <int BS>
+constexpr int brows_at_once() { return BS >= 1024 ? 1 : 4; }
+
+// use(i, s) for every row i of the workgroup's system in the thread's order,
+// s = row of A*v in column order (mat_vec_mult.hpp:656-682).  The indices and
+// values of up to eight entries of each of the rows are requested together,
+// then their gathers: as many as the longest row of the wave has left (each
+// load of a row per lane is 64 places for the memory unit: always eight cost
+// 1024 threads a fifth more than they gained).  Entries past a lane's row
+// reload its last one and are dropped.
+template <int BS, typename AT, typename MT, typename VT, typename F>
+__device__ __forceinline__ void brows(const BatchDev& M, const MT* __restrict__ val, int r0, int n,
+                                      const VT* __restrict__ v, F use) {
+    constexpr int U = brows_at_once<BS>();
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * BS) {
+        int j0[U], j1[U];
+        AT s[U];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const bool in = j + u < j1;
-            c[u] = in ? M.col[j + u] - r0 : 0;
-            m[u] = in ? load_val<AT>(val, j + u) : AT(0);
+        for (int u = 0; u < U; u++) {
+            const int row = r0 + min(i0 + u * BS, n - 1);
+            j0[u] = M.rowptr[row];
+            j1[u] = M.rowptr[row + 1];
+            s[u] = AT(0);
+        }
+        for (bool more = true; more;) {
+            int c[U][8];
+            AT m[U][8], g[U][8];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    c[u][e] = r0;
+                    m[u][e] = AT(0);
+                    if (__any(j0[u] + e < j1[u])) {
+                        const int j = max(min(j0[u] + e, j1[u] - 1), 0);
+                        c[u][e] = M.col[j];
+                        m[u][e] = load_val<AT>(val, j);
+                    }
+                }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    g[u][e] = AT(0);
+                    if (__any(j0[u] + e < j1[u])) g[u][e] = static_cast<AT>(v[j0[u] + e < j1[u] ? c[u][e] - r0 : 0]);
+                }
+            more = false;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const AT with = s[u] + m[u][e] * g[u][e];
+                    s[u] = j0[u] + e < j1[u] ? with : s[u];
+                }
+                j0[u] += 8;
+                more |= j0[u] < j1[u];
+            }
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) g[u] = j + u < j1 ? static_cast<AT>(v[c[u]]) : AT(0);
-#pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (j + u < j1) s += m[u] * g[u];
+        for (int u = 0; u < U; u++)
+            if (i0 + u * BS < n) use(i0 + u * BS, s[u]);
     }
-    return s;
 }
+
+// store(i, load(i)) for every element i in the thread's order, the loads of
+// several elements first.
+template <int BS, typename L, typename F>
+__device__ __forceinline__ void belems(int n, L load, F store) {
+    constexpr int U = brows_at_once<BS>();
+    int i = threadIdx.x;
+    for (; i + (U - 1) * BS < n; i += U * BS) {
+        decltype(load(0)) in[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) in[u] = load(i + u * BS);
+#pragma unroll
+        for (int u = 0; u < U; u++) store(i + u * BS, in[u]);
+    }
+    for (; i < n; i += BS) store(i, load(i));
+}
+template <typename T, int N>
+struct BIn {
+    T v[N];
+};
 
 __device__ __forceinline__ bool bconv(double resid, double norm_r0, double rtol, double atol) {
     return norm_r0 == 0 ? resid <= atol : (resid <= rtol * norm_r0 || resid <= atol);
@@ -92,36 +160,104 @@ __device__ __forceinline__ int next_item(unsigned* queue, int* s_k) {
 // One level-scheduled triangular sweep of system `sys` inside its workgroup:
 // w[r] = (v[r] - sum_j T[r][c_j] * w[c_j]) [* dia], each row in MTL4's
 // subtraction order (lower_trisolve.hpp:174-189 unit, upper_trisolve.hpp:
-// 161-176 inverse diagonal first), a barrier between levels.  v and w are
-// the system's local vectors; w is read back only after a barrier.
+// 161-176 inverse diagonal first), a barrier between levels.  v may be w
+// itself (a row's input is read before its result is written); w is read back
+// only after a barrier.
+//
+// What bounds it: a row's five dependent round trips (level, place, bounds,
+// entries, neighbours) once per level, about 2 us.  All but the last do not
+// depend on the levels before, so a thread requests the places of its row two
+// levels ahead and its entries one level ahead (its first kSweepAhead entries;
+// levels wider than the workgroup and longer rows do the rest in place).
+constexpr int kSweepAhead = 4;
 template <int BS, bool UNIT, typename VT>
 __device__ __forceinline__ void bsweep(const BatchSweepDev& S, const VT* __restrict__ val,
                                        const VT* __restrict__ dia, int sys, int r0,
                                        const double* v, double* w) {
-    const int l0 = S.lev_off[sys], l1 = S.lev_off[sys + 1] - 1;
-    for (int l = l0; l < l1; l++) {
-        const int a = S.lev[l], e = S.lev[l + 1];
-        for (int k = a + (int)threadIdx.x; k < e; k += BS) {
-            const int lr = S.perm[k] - r0;
-            double acc = v[lr];
-            const int j1 = S.rowptr[k + 1];
-            for (int j = S.rowptr[k]; j < j1; j++) acc -= (double)val[j] * w[S.col[j] - r0];
-            if (!UNIT) acc = acc * (double)dia[k];
-            w[lr] = acc;
+    const int l0 = S.lev_off[sys], l1 = S.lev_off[sys + 1] - 1, t = (int)threadIdx.x;
+    struct Place {
+        int k, lr, j0, j1;   // k < 0: no row
+    };
+    struct Row {
+        int lr, j0, j1, c[kSweepAhead];
+        double m[kSweepAhead], d;
+    };
+    auto place = [&](int l) {
+        Place p{-1, 0, 0, 0};
+        if (l < l1) {
+            const int k = S.lev[l] + t;
+            if (k < S.lev[l + 1]) {
+                p.k = k;
+                p.lr = S.perm[k] - r0;
+                p.j0 = S.rowptr[k];
+                p.j1 = S.rowptr[k + 1];
+            }
         }
+        return p;
+    };
+    auto row = [&](const Place& p) {
+        Row r{p.lr, p.j0, p.j1, {}, {}, 1.0};
+        if (p.k >= 0) {
+            if (!UNIT) r.d = (double)dia[p.k];
+#pragma unroll
+            for (int e = 0; e < kSweepAhead; e++) {
+                const int j = max(min(p.j0 + e, p.j1 - 1), 0);   // past the row's end: a valid entry, dropped
+                r.c[e] = S.col[j] - r0;
+                r.m[e] = (double)val[j];
+            }
+        }
+        return r;
+    };
+    auto solve = [&](const Row& r) {
+        double acc = v[r.lr], g[kSweepAhead];
+#pragma unroll
+        for (int e = 0; e < kSweepAhead; e++) g[e] = w[r.j0 + e < r.j1 ? r.c[e] : r.lr];
+#pragma unroll
+        for (int e = 0; e < kSweepAhead; e++) {
+            const double next = acc - r.m[e] * g[e];
+            acc = r.j0 + e < r.j1 ? next : acc;
+        }
+        for (int j = r.j0 + kSweepAhead; j < r.j1; j++) acc -= (double)val[j] * w[S.col[j] - r0];
+        if (!UNIT) acc = acc * r.d;
+        w[r.lr] = acc;
+    };
+    Place p = place(l0), ahead = place(l0 + 1);
+    Row r = row(p);
+    for (int l = l0; l < l1; l++) {
+        const Place later = place(l + 2);
+        const Row next = row(ahead);
+        if (p.k >= 0) solve(r);
+        for (int k = S.lev[l] + t + BS; k < S.lev[l + 1]; k += BS)   // a level wider than the workgroup
+            solve(row(Place{k, S.perm[k] - r0, S.rowptr[k], S.rowptr[k + 1]}));
         __syncthreads();
+        p = ahead;
+        ahead = later;
+        r = next;
     }
 }
 
-// z = solve(ilu_0, r): unit lower sweep into y, upper sweep into z
+// z = solve(ilu_0, r): unit lower sweep, upper sweep.  Systems of up to
+// kSweepLds rows sweep in LDS (in place: a row's input is its own slot), larger
+// ones through y and z.
+constexpr int kSweepLds = 4096;
 template <int BS, bool LOW>
-__device__ __forceinline__ void bilu(const BatchDev& M, int sys, int r0, const double* r, double* y, double* z) {
-    if (LOW) {
-        bsweep<BS, true>(M.lo, M.lo.val32, M.lo.dia32, sys, r0, r, y);
-        bsweep<BS, false>(M.up, M.up.val32, M.up.dia32, sys, r0, y, z);
+__device__ __forceinline__ void bilu(const BatchDev& M, int sys, int r0, int n, const double* r, double* y, double* z,
+                                     double* lds) {
+    auto both = [&](const double* in, double* mid, double* out) {
+        if (LOW) {
+            bsweep<BS, true>(M.lo, M.lo.val32, M.lo.dia32, sys, r0, in, mid);
+            bsweep<BS, false>(M.up, M.up.val32, M.up.dia32, sys, r0, mid, out);
+        } else {
+            bsweep<BS, true>(M.lo, M.lo.val, M.lo.dia, sys, r0, in, mid);
+            bsweep<BS, false>(M.up, M.up.val, M.up.dia, sys, r0, mid, out);
+        }
+    };
+    if (n <= kSweepLds) {
+        both(r, lds, lds);
+        for (int i = threadIdx.x; i < n; i += BS) z[i] = lds[i];
+        __syncthreads();
     } else {
-        bsweep<BS, true>(M.lo, M.lo.val, M.lo.dia, sys, r0, r, y);
-        bsweep<BS, false>(M.up, M.up.val, M.up.dia, sys, r0, y, z);
+        both(r, y, z);
     }
 }
 
@@ -145,6 +281,7 @@ __global__ __launch_bounds__(BS) void k_batch_cg64(BatchDev M, const MT* __restr
                                                    double* W, mtl4g_batch_result* out, double delta) {
     constexpr bool LOW = !std::is_same<MT, double>::value;
     __shared__ double sh[2 * (BS / kWave)];
+    __shared__ double sweep[PCM == BPC_ILU ? kSweepLds : 1];
     __shared__ int s_k;
     for (;;) {
         const int k = next_item(queue, &s_k);
@@ -162,14 +299,14 @@ __global__ __launch_bounds__(BS) void k_batch_cg64(BatchDev M, const MT* __restr
         auto dv = [&](int i) -> double { return LOW ? (double)M.dinv32[r0 + i] : M.dinv[r0 + i]; };
         // basic_iteration(b, ...): norm_r0 = two_norm(b); r = b - A*x; rr, rho
         double bb = 0, rr = 0, rho = 0, tmp = 0;
-        for (int i = threadIdx.x; i < n; i += BS) {
+        brows<BS, double>(M, M.val, r0, n, x, [&](int i, double s) {
             const double bi = b[i];
             bb += bi * bi;
-            const double v = bi - brow<double>(M, M.val, r0 + i, r0, x);
+            const double v = bi - s;
             r[i] = v;
             rr += v * v;
             if (PCM == BPC_DIAG) rho += v * (dv(i) * v);
-        }
+        });
         block_sum2<BS>(bb, rr, sh);
         if (PCM == BPC_DIAG) block_sum2<BS>(rho, tmp, sh);
         else rho = rr;
@@ -186,12 +323,12 @@ __global__ __launch_bounds__(BS) void k_batch_cg64(BatchDev M, const MT* __restr
                     restart = !isfinite(resid) || grown;
                     rr = 0;
                     rho = 0;
-                    for (int i = threadIdx.x; i < n; i += BS) {
-                        const double v = b[i] - brow<double>(M, M.val, r0 + i, r0, x);
+                    brows<BS, double>(M, M.val, r0, n, x, [&](int i, double s) {
+                        const double v = b[i] - s;
                         r[i] = v;
                         rr += v * v;
                         if (PCM == BPC_DIAG) rho += v * (dv(i) * v);
-                    }
+                    });
                     block_sum2<BS>(rr, rho, sh);
                     if (PCM != BPC_DIAG) rho = rr;
                     resid = sqrt(fabs(rr));
@@ -209,38 +346,46 @@ __global__ __launch_bounds__(BS) void k_batch_cg64(BatchDev M, const MT* __restr
             const bool first = iters <= 1 || restart;
             restart = false;
             if (PCM == BPC_ILU) {   // z = solve(P, r); rho = dot(r, z)
-                bilu<BS, LOW>(M, it.sys, r0, r, y, z);
+                bilu<BS, LOW>(M, it.sys, r0, n, r, y, z, sweep);
                 double rz = 0;
                 tmp = 0;
-                for (int i = threadIdx.x; i < n; i += BS) rz += r[i] * z[i];
+                belems<BS>(n, [&](int i) { return BIn<double, 2>{r[i], z[i]}; },
+                           [&](int, const BIn<double, 2>& e) { rz += e.v[0] * e.v[1]; });
                 block_sum2<BS>(rz, tmp, sh);
                 rho = rz;
             }
             const double beta = first ? 0.0 : rho / rho_1;
-            for (int i = threadIdx.x; i < n; i += BS) {   // p = z + beta*p
-                const double zi = PCM == BPC_DIAG ? dv(i) * r[i] : PCM == BPC_ILU ? z[i] : r[i];
-                p[i] = first ? zi : zi + beta * p[i];
-            }
+            belems<BS>(   // p = z + beta*p
+                n,
+                [&](int i) {
+                    return BIn<double, 2>{PCM == BPC_DIAG ? dv(i) * r[i] : PCM == BPC_ILU ? z[i] : r[i],
+                                          first ? 0.0 : p[i]};
+                },
+                [&](int i, const BIn<double, 2>& e) { p[i] = first ? e.v[0] : e.v[0] + beta * e.v[1]; });
             __syncthreads();
             double pq = 0;
             tmp = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // q = A*p, p.q
-                const double s = brow<double>(M, aval, r0 + i, r0, p);
+            brows<BS, double>(M, aval, r0, n, p, [&](int i, double s) {   // q = A*p, p.q
                 q[i] = s;
                 pq += p[i] * s;
-            }
+            });
             block_sum2<BS>(pq, tmp, sh);
             const double alpha = rho / pq;
             rho_1 = rho;
             rr = 0;
             double rhon = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // x += alpha p; r -= alpha q
-                x[i] = x[i] + alpha * p[i];
-                const double v = r[i] - alpha * q[i];
-                r[i] = v;
-                rr += v * v;
-                if (PCM == BPC_DIAG) rhon += v * (dv(i) * v);
-            }
+            belems<BS>(   // x += alpha p; r -= alpha q
+                n,
+                [&](int i) {
+                    return BIn<double, 5>{x[i], p[i], r[i], q[i], PCM == BPC_DIAG ? dv(i) : 0.0};
+                },
+                [&](int i, const BIn<double, 5>& e) {
+                    x[i] = e.v[0] + alpha * e.v[1];
+                    const double v = e.v[2] - alpha * e.v[3];
+                    r[i] = v;
+                    rr += v * v;
+                    if (PCM == BPC_DIAG) rhon += v * (e.v[4] * v);
+                });
             block_sum2<BS>(rr, rhon, sh);
             resid = sqrt(fabs(rr));
             rho = PCM == BPC_DIAG ? rhon : rr;
@@ -263,6 +408,7 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
     constexpr bool LOW = !std::is_same<MT, double>::value;
     (void)delta;   // BiCGSTAB refreshes at kBatchBicgDelta
     __shared__ double sh[2 * (BS / kWave)];
+    __shared__ double sweep[PCM == BPC_ILU ? kSweepLds : 1];
     __shared__ int s_k;
     for (;;) {
         const int k = next_item(queue, &s_k);
@@ -288,22 +434,22 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
         auto dv = [&](int i) -> double { return LOW ? (double)M.dinv32[r0 + i] : M.dinv[r0 + i]; };
         auto pc = [&](const double* in, double* o) {
             if (PCM == BPC_DIAG) {
-                for (int i = threadIdx.x; i < n; i += BS) o[i] = dv(i) * in[i];
+                belems<BS>(n, [&](int i) { return dv(i) * in[i]; }, [&](int i, double e) { o[i] = e; });
                 __syncthreads();
             } else if (PCM == BPC_ILU) {
-                bilu<BS, LOW>(M, it.sys, r0, in, y, o);
+                bilu<BS, LOW>(M, it.sys, r0, n, in, y, o, sweep);
             }
         };
         // r = b - A*x; rtilde = r
         double bb = 0, rr = 0;
-        for (int i = threadIdx.x; i < n; i += BS) {
+        brows<BS, double>(M, M.val, r0, n, x, [&](int i, double s) {
             const double bi = b[i];
             bb += bi * bi;
-            const double vv = bi - brow<double>(M, M.val, r0 + i, r0, x);
+            const double vv = bi - s;
             r[i] = vv;
             rt[i] = vv;
             rr += vv * vv;
-        }
+        });
         block_sum2<BS>(bb, rr, sh);
         const double norm_r0 = sqrt(bb);
         double resid = sqrt(fabs(rr)), rmax = resid;
@@ -320,12 +466,12 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
                     restart = true;
                     rr = 0;
                     double tmp = 0;
-                    for (int i = threadIdx.x; i < n; i += BS) {
-                        const double vv = b[i] - brow<double>(M, M.val, r0 + i, r0, x);
+                    brows<BS, double>(M, M.val, r0, n, x, [&](int i, double s) {
+                        const double vv = b[i] - s;
                         r[i] = vv;
                         rt[i] = vv;
                         rr += vv * vv;
-                    }
+                    });
                     block_sum2<BS>(rr, tmp, sh);
                     resid = sqrt(fabs(rr));
                     rmax = resid;
@@ -342,7 +488,8 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
             const bool first = iters <= 1 || restart;
             restart = false;
             double rho_1 = 0, tmp = 0;
-            for (int i = threadIdx.x; i < n; i += BS) rho_1 += rt[i] * r[i];
+            belems<BS>(n, [&](int i) { return BIn<double, 2>{rt[i], r[i]}; },
+                       [&](int, const BIn<double, 2>& e) { rho_1 += e.v[0] * e.v[1]; });
             block_sum2<BS>(rho_1, tmp, sh);
             if (rho_1 == 0.0) { status = MTL4G_ERR_BREAKDOWN; break; }
             double beta = 0;
@@ -350,26 +497,31 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
                 if (omega == 0.0) { status = MTL4G_ERR_BREAKDOWN; break; }
                 beta = (rho_1 / rho_2) * (alpha / omega);
             }
-            for (int i = threadIdx.x; i < n; i += BS) p[i] = first ? r[i] : r[i] + beta * (p[i] - omega * v[i]);
+            belems<BS>(
+                n, [&](int i) { return BIn<double, 3>{r[i], first ? 0.0 : p[i], first ? 0.0 : v[i]}; },
+                [&](int i, const BIn<double, 3>& e) {
+                    p[i] = first ? e.v[0] : e.v[0] + beta * (e.v[1] - omega * e.v[2]);
+                });
             __syncthreads();
             pc(p, ph);
             double gamma = 0;
             tmp = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // v = A*phat; gamma = dot(rtilde, v)
-                const double s = brow<double>(M, aval, r0 + i, r0, ph);
+            brows<BS, double>(M, aval, r0, n, ph, [&](int i, double s) {   // v = A*phat; gamma = dot(rtilde, v)
                 v[i] = s;
                 gamma += rt[i] * s;
-            }
+            });
             block_sum2<BS>(gamma, tmp, sh);
             if (gamma == 0.0) { status = MTL4G_ERR_BREAKDOWN; break; }
             alpha = rho_1 / gamma;
             double ss = 0;
             tmp = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // s = r - alpha*v
-                const double si = r[i] - alpha * v[i];
-                sv[i] = si;
-                ss += si * si;
-            }
+            belems<BS>(   // s = r - alpha*v
+                n, [&](int i) { return BIn<double, 2>{r[i], v[i]}; },
+                [&](int i, const BIn<double, 2>& e) {
+                    const double si = e.v[0] - alpha * e.v[1];
+                    sv[i] = si;
+                    ss += si * si;
+                });
             block_sum2<BS>(ss, tmp, sh);
             const double sres = sqrt(ss);
             const bool half_stop = LOW ? (!isfinite(sres) || bconv(sres, norm_r0, it.rtol, it.atol))
@@ -392,21 +544,22 @@ __global__ __launch_bounds__(BS) void k_batch_bicg64(BatchDev M, const MT* __res
             }
             pc(sv, shv);
             double ts = 0, tt = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // t = A*shat; omega = dot(t,s)/dot(t,t)
-                const double ti = brow<double>(M, aval, r0 + i, r0, shv);
+            brows<BS, double>(M, aval, r0, n, shv, [&](int i, double ti) {   // t = A*shat; omega = dot(t,s)/dot(t,t)
                 t[i] = ti;
                 ts += ti * sv[i];
                 tt += ti * ti;
-            }
+            });
             block_sum2<BS>(ts, tt, sh);
             omega = ts / tt;
             rr = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {   // x += omega*shat + alpha*phat; r = s - omega*t
-                x[i] = x[i] + (omega * shv[i] + alpha * ph[i]);
-                const double ri = sv[i] - omega * t[i];
-                r[i] = ri;
-                rr += ri * ri;
-            }
+            belems<BS>(   // x += omega*shat + alpha*phat; r = s - omega*t
+                n, [&](int i) { return BIn<double, 5>{x[i], shv[i], ph[i], sv[i], t[i]}; },
+                [&](int i, const BIn<double, 5>& e) {
+                    x[i] = e.v[0] + (omega * e.v[1] + alpha * e.v[2]);
+                    const double ri = e.v[3] - omega * e.v[4];
+                    r[i] = ri;
+                    rr += ri * ri;
+                });
             tmp = 0;
             block_sum2<BS>(rr, tmp, sh);
             resid = sqrt(fabs(rr));
@@ -452,19 +605,20 @@ __global__ __launch_bounds__(BS) void k_batch_mixed(BatchDev M, const MT* __rest
         float rho = 0;
         int refreshes = 0;
         auto refresh = [&]() {
-            for (int i = threadIdx.x; i < n; i += BS) {
-                x[i] = x[i] + (double)x32[i];
-                x32[i] = 0.0f;
-            }
+            belems<BS>(n, [&](int i) { return BIn<double, 2>{x[i], (double)x32[i]}; },
+                       [&](int i, const BIn<double, 2>& e) {
+                           x[i] = e.v[0] + e.v[1];
+                           x32[i] = 0.0f;
+                       });
             __syncthreads();
             double r2 = 0, rz = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {
-                const double v = b[i] - brow<double>(M, M.val, r0 + i, r0, x);
+            brows<BS, double>(M, M.val, r0, n, x, [&](int i, double s) {
+                const double v = b[i] - s;
                 const float f = (float)v;
                 r[i] = f;
                 r2 += v * v;
                 rz += PCM == BPC_DIAG ? (double)(f * (d[i] * f)) : (double)(f * f);
-            }
+            });
             block_sum2<BS>(r2, rz, sh);
             resid64 = sqrt(r2);
             rho = (float)rz;
@@ -497,28 +651,28 @@ __global__ __launch_bounds__(BS) void k_batch_mixed(BatchDev M, const MT* __rest
             iters++;
             const bool first = iters <= 1;
             const float beta = first ? 0.0f : rho / rho_1;
-            for (int i = threadIdx.x; i < n; i += BS) {
-                const float zi = PCM == BPC_DIAG ? d[i] * r[i] : r[i];
-                p[i] = first ? zi : zi + beta * p[i];
-            }
+            belems<BS>(
+                n, [&](int i) { return BIn<float, 2>{PCM == BPC_DIAG ? d[i] * r[i] : r[i], first ? 0.0f : p[i]}; },
+                [&](int i, const BIn<float, 2>& e) { p[i] = first ? e.v[0] : e.v[0] + beta * e.v[1]; });
             __syncthreads();
             float pq = 0, tf = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {
-                const float s = brow<float>(M, val32, r0 + i, r0, p);
+            brows<BS, float>(M, val32, r0, n, p, [&](int i, float s) {
                 q[i] = s;
                 pq += p[i] * s;
-            }
+            });
             block_sum2<BS>(pq, tf, shf);
             const float alpha = rho / pq;
             rho_1 = rho;
             float rr = 0, rhon = 0;
-            for (int i = threadIdx.x; i < n; i += BS) {
-                x32[i] = x32[i] + alpha * p[i];
-                const float v = r[i] - alpha * q[i];
-                r[i] = v;
-                rr += v * v;
-                if (PCM == BPC_DIAG) rhon += v * (d[i] * v);
-            }
+            belems<BS>(
+                n, [&](int i) { return BIn<float, 5>{x32[i], p[i], r[i], q[i], PCM == BPC_DIAG ? d[i] : 0.0f}; },
+                [&](int i, const BIn<float, 5>& e) {
+                    x32[i] = e.v[0] + alpha * e.v[1];
+                    const float v = e.v[2] - alpha * e.v[3];
+                    r[i] = v;
+                    rr += v * v;
+                    if (PCM == BPC_DIAG) rhon += v * (e.v[4] * v);
+                });
             block_sum2<BS>(rr, rhon, shf);
             resid32 = sqrt(fabs((double)rr));
             rho = PCM == BPC_DIAG ? rhon : rr;
