@@ -1,4 +1,4 @@
-// resident.hpp -- itl::cg with its state on the chip (resident.hip).
+// resident.hpp -- itl::cg with its state on the chip (resident.hip, resident_large.hip).
 #pragma once
 
 #include "krylov.hpp"
@@ -22,12 +22,14 @@ int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
 struct ResidentPlan {
     int op = 0;          // 0: not taken; else the kernel variant
     int rows_log2 = 0;   // rows per lane: 1 << rows_log2
+    int groups = 0;      // streamed matrix: 16-byte groups of rows per lane
     int grid = 0;        // workgroups
     int halo = 0;        // diagonal operand: neighbouring elements kept in LDS
     int neigh = 0;       // workgroups on either side whose p is read
     bool share = false;  // p goes through memory
 };
-ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes);
+// vectors of vt_bytes per element; own_diag: no inverse diagonal, or one in the vectors' type
+ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_format, bool own_diag);
 template <typename VT>
 int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
                     int dfmt, Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s);
@@ -54,7 +56,8 @@ int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
                 hipStream_t s, int32_t steps, After after, bool* ran) {
     *ran = false;
     if (W.shared_gpu) return MTL4G_OK;
-    const ResidentPlan plan = resident_plan(A, (int)sizeof(VT));
+    const ResidentPlan plan = resident_plan(
+        A, (int)sizeof(VT), value_format, !inv_diag || dfmt == (sizeof(VT) == 8 ? MTL4G_F64 : MTL4G_F32));
     if (!plan.op) return MTL4G_OK;
     int launches = 1;
     for (;;) {
