@@ -73,7 +73,7 @@ __global__ void k_fill_pending(int64_t n, VT* w, const int* skip) {
 // v (input, type IT) and w are distinct arrays; w holds the results in VT,
 // the type the row arithmetic runs in, and w32 (may be null) receives each
 // result rounded to float as well.
-template <int BS, typename MT, typename IT, typename VT>
+template <int BS, int E, typename MT, typename IT, typename VT>
 __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __restrict__ v,
                                               VT* w, float* w32, unsigned* counters, int* err,
                                               const int* skip) {
@@ -85,14 +85,14 @@ __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __r
     const int b = s_b;
     const int L = S.blk_level[b];
     // The row's own data (position, bounds, right-hand side, diagonal and its
-    // first eight entries) does not depend on earlier levels: request it
+    // first E entries) does not depend on earlier levels: request it
     // before waiting.
     const int k = S.lev_ptr[L] + (b - S.lev_blk[L]) * BS + (int)threadIdx.x;
     const bool mine = k < S.lev_ptr[L + 1];
     int r = 0, a = 0, e = 0;
     VT rr = VT(0), dk = VT(1);
-    int c[8];
-    VT m[8];
+    int c[E];
+    VT m[E];
     if (mine) {
         r = S.perm[k];
         a = S.rowptr[k];
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __r
         rr = static_cast<VT>(v[r]);
         if (!S.unit) dk = to_arith<VT>(S.dia[k]);
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < E; u++) {
             const bool in = a + u < e;
             c[u] = in ? S.col[a + u] : 0;
             m[u] = in ? to_arith<VT>(S.val[a + u]) : VT(0);
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __r
             while (ld_agent(lev) < need) {
                 if ((++it & 63u) == 0 && ld_agent(sweep_counter(counters, 1)) != 0u) { ok = 0; break; }
                 if (it > kSpinLimit) { st_agent(sweep_counter(counters, 1), 1u); ok = 0; break; }
-                __builtin_amdgcn_s_sleep(2);
+                __builtin_amdgcn_s_sleep(8);   // 2: 223 instead of 214 us on the graph below (launch_levels)
             }
         }
         s_ok = ok;
@@ -123,26 +123,26 @@ __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __r
     __syncthreads();
     if (s_ok && mine) {
         bool ok = true;
-        // eight entries at a time: the eight values they name (one round
+        // E entries at a time: the values they name (one round
         // trip, repeated for those still pending), then the subtractions in
         // the row's column order
-        for (int j0 = a; j0 < e && ok; j0 += 8) {
+        for (int j0 = a; j0 < e && ok; j0 += E) {
             if (j0 > a) {
 #pragma unroll
-                for (int u = 0; u < 8; u++) {
+                for (int u = 0; u < E; u++) {
                     const bool in = j0 + u < e;
                     c[u] = in ? S.col[j0 + u] : 0;
                     m[u] = in ? to_arith<VT>(S.val[j0 + u]) : VT(0);
                 }
             }
-            VT wv[8];
+            VT wv[E];
 #pragma unroll
-            for (int u = 0; u < 8; u++) wv[u] = j0 + u < e ? ld_agent(w + c[u]) : VT(0);
+            for (int u = 0; u < E; u++) wv[u] = j0 + u < e ? ld_agent(w + c[u]) : VT(0);
             unsigned it = 0;
             for (;;) {
                 bool wait = false;
 #pragma unroll
-                for (int u = 0; u < 8; u++) wait |= pending(wv[u]);
+                for (int u = 0; u < E; u++) wait |= pending(wv[u]);
                 if (!wait) break;
                 if (++it > kSpinLimit) {
                     st_agent(sweep_counter(counters, 1), 1u);
@@ -155,11 +155,11 @@ __global__ __launch_bounds__(BS) void k_sweep(SweepView<MT, VT> S, const IT* __r
                 }
                 __builtin_amdgcn_s_sleep(1);
 #pragma unroll
-                for (int u = 0; u < 8; u++)
+                for (int u = 0; u < E; u++)
                     if (pending(wv[u])) wv[u] = ld_agent(w + c[u]);
             }
 #pragma unroll
-            for (int u = 0; u < 8; u++)
+            for (int u = 0; u < E; u++)
                 if (j0 + u < e) rr -= m[u] * wv[u];
         }
         if (!S.unit) rr = rr * dk;
@@ -710,6 +710,26 @@ size_t Sweep::words() const {
     return chain_counter_words + 2 * (size_t)(chain->xtile * chain->tiles_x * chain->tiles_y);
 }
 
+template <typename MT, typename IT, typename VT>
+static void launch_levels(const Sweep& S, const MT* val, const MT* dia, const IT* v, VT* w, float* w32,
+                          unsigned* counters, int* err, const int* skip, hipStream_t s) {
+    const SweepView<MT, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
+                              S.blk_level.p, val, dia, S.nlev, S.unit ? 1 : 0};
+    const dim3 grid(S.nblocks), block(kSweepBS);
+    // Entries requested before the wait: a row with more pays another round trip
+    // on its level's path, one with fewer issues the loads for nothing.  Two
+    // sweeps of a graph's factor (120,011 rows, 5.5 entries per row, up to 16 and
+    // more): 265 us with 4, 234 with 8, 222 with 16; of a 5-point factor
+    // (90,000 rows, 2 entries): 1129, 1226 and 1581 us.  The line between lies
+    // where a row of the mean length and a few more still fits.
+    if (S.nnz <= 3 * (int64_t)S.n)
+        hipLaunchKernelGGL((k_sweep<kSweepBS, 4, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
+    else if (S.nnz <= 4 * (int64_t)S.n)
+        hipLaunchKernelGGL((k_sweep<kSweepBS, 8, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
+    else
+        hipLaunchKernelGGL((k_sweep<kSweepBS, 16, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
+}
+
 template <typename IT, typename VT>
 int launch_sweep(const Sweep& S, int fmt, const IT* v, VT* w, float* w32, const int* skip, int* err,
                  unsigned* counters, hipStream_t s) {
@@ -720,22 +740,9 @@ int launch_sweep(const Sweep& S, int fmt, const IT* v, VT* w, float* w32, const 
         return launch_chain<IT>(*S.chain, fmt, v, w, w32, counters, err, skip, s);
     }
     hipLaunchKernelGGL(k_fill_pending<VT>, dim3(grid_for(S.n)), dim3(256), 0, s, (int64_t)S.n, w, skip);
-    if (fmt == MTL4G_F64) {
-        SweepView<double, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
-                                S.blk_level.p, S.val64.p, S.dia64.p, S.nlev, S.unit ? 1 : 0};
-        hipLaunchKernelGGL((k_sweep<kSweepBS, double, IT, VT>), dim3(S.nblocks), dim3(kSweepBS), 0, s,
-                           V, v, w, w32, counters, err, skip);
-    } else if (fmt == MTL4G_F32) {
-        SweepView<float, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
-                               S.blk_level.p, S.val32.p, S.dia32.p, S.nlev, S.unit ? 1 : 0};
-        hipLaunchKernelGGL((k_sweep<kSweepBS, float, IT, VT>), dim3(S.nblocks), dim3(kSweepBS), 0, s,
-                           V, v, w, w32, counters, err, skip);
-    } else {
-        SweepView<uint16_t, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
-                                  S.blk_level.p, S.val16.p, S.dia16.p, S.nlev, S.unit ? 1 : 0};
-        hipLaunchKernelGGL((k_sweep<kSweepBS, uint16_t, IT, VT>), dim3(S.nblocks), dim3(kSweepBS), 0, s,
-                           V, v, w, w32, counters, err, skip);
-    }
+    if (fmt == MTL4G_F64) launch_levels(S, S.val64.p, S.dia64.p, v, w, w32, counters, err, skip, s);
+    else if (fmt == MTL4G_F32) launch_levels(S, S.val32.p, S.dia32.p, v, w, w32, counters, err, skip, s);
+    else launch_levels(S, S.val16.p, S.dia16.p, v, w, w32, counters, err, skip, s);
     M4_HIP(hipGetLastError());
     return MTL4G_OK;
 }
