@@ -921,7 +921,8 @@ def main():
         "cg_iteration": {"us": round(1e6 * t_fp64 / args.steps / max(iters, 1), 2),
                          "bytes": it_bytes, "GBs": round(it_bytes * iters * args.steps / t_fp64 / 1e9, 1),
                          "frac": round(it_bytes * iters * args.steps / t_fp64 / 1e9 / HBM_PEAK_GBS, 4),
-                         "note": "the layout's SpMV bytes + 11 vector passes (P: 4, XR: 7) per iteration"},
+                         "note": "the layout's SpMV bytes + 11 vector passes (P: 4, XR: 7): the bytes of the "
+                                 "launch-per-kernel loop; a solve kept on the chip moves fewer"},
         "spmv": {"diffusion3d_f64_GBs": round(ctx_gbs, 1), "diffusion3d_f64_back_to_back_GBs": round(spmv_gbs, 1),
                  "random_2M_poisson16_f64_GBs": round(rnd_gbs, 1),
                  "random_frac_of_peak": round(rnd_gbs / HBM_PEAK_GBS, 4)},

@@ -126,7 +126,9 @@ int mtl4g_get_reduction_order(void);
  * iterations (at most 65536 per solve); mtl4g_product_timing returns the
  * summed duration in microseconds and the number of products of the solves
  * since the last call (launches past a solve's stop are not counted), and
- * clears them.  Process-wide; for one solve at a time. */
+ * clears them.  A CG solve that keeps its state on the chip (many iterations
+ * per launch) runs one iteration per launch meanwhile, with the product
+ * launched and timed beside it.  Process-wide; for one solve at a time. */
 int mtl4g_set_product_timing(int on);
 int mtl4g_product_timing(double* h_total_us, int64_t* h_count);
 

@@ -9,7 +9,9 @@
 // host only enqueues chunks of iterations and polls Ctl::done between
 // chunks; no host round trip sits inside an iteration.
 //
-// CG + diagonal (cg.hpp:74-111) runs three kernels per iteration:
+// CG + identity / diagonal runs on the chip where the matrix allows it
+// (resident.hip, resident_large.hip); otherwise, and in MTL4's order, CG +
+// diagonal (cg.hpp:74-111) runs three kernels per iteration:
 //   P : p = z + beta*p            with z = inv_diag .* r formed on the fly
 //   Q : q = A*p, p.q              (SpMV + dot, cg.hpp:103)      -> alpha
 //   XR: x += alpha*p, r -= alpha*q, r.r, r.(inv_diag .* r)      -> stop?, beta
