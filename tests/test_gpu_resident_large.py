@@ -93,3 +93,27 @@ def test_large_mixed_cg(m, sizes, layout, fmt):
         assert err == 0 and st["relres"] <= 1e-10
         r = b.numpy() - (A * x).numpy()
         assert np.linalg.norm(r) <= 1.01e-10 * np.linalg.norm(b.numpy())
+
+
+@pytest.mark.parametrize("sizes", [(102, 104, 102), (160, 160, 160)])
+def test_large_cg_vectors_off_a_16_byte_boundary(m, sizes):
+    """x and b that start 8 bytes past one: the same bits."""
+    import torch
+    rp, ci, va = _grid(sizes)
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    A.set_kernel(m._lib.SPMV_DIA_SYM, 4, 4)
+    P = m.pc.diagonal(A)
+    b = A * m.dense_vector(np.random.default_rng(5).uniform(-1, 1, n))
+    xs = []
+    for shift in (0, 1):
+        print("large cg shifted", sizes, shift, flush=True)
+        buf = torch.zeros(n + 2, dtype=torch.float64, device="cuda")
+        bb = torch.zeros(n + 2, dtype=torch.float64, device="cuda")
+        bb[shift:shift + n] = b.t
+        x, bd = m.dense_vector(buf[shift:shift + n]), m.dense_vector(bb[shift:shift + n])
+        assert x.t.data_ptr() % 16 == 8 * shift
+        m.cg(A, x, bd, P, m.basic_iteration(bd, 6, 0.0))
+        xs.append(x.numpy().copy())
+        assert float(buf[:shift].abs().sum() + buf[shift + n:].abs().sum()) == 0.0
+    assert np.array_equal(xs[0], xs[1])
