@@ -15,7 +15,7 @@
 // (p, q, x, r; rows summed in column order); the sums are combined in another
 // fixed order, which depends only on the system, so a solve is deterministic.
 //
-// Workgroups wait for each other (Sync below), so all of them must be on the
+// Workgroups wait for each other (resident_dev.hpp), so all of them must be on the
 // chip at once.  A launch first meets at a rendezvous with a bounded wait:
 // when the grid does not get onto the chip (another kernel holds its CUs) the
 // launch gives up before it has changed anything and the host tries again.
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(kResBS) void k_cg_resident(ResArgs a) {
 // Slots pending, words zero, before each launch.
 __global__ void k_resident_begin(ResSync S) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 3 * kSlotGen) S.slots[i] = __longlong_as_double((long long)kResPending);
+    if (i < kSlotGens * kSlotGen) S.slots[i] = __longlong_as_double((long long)kResPending);
     if (i < kResWords) S.words[i] = 0u;
 }
 
@@ -479,7 +479,7 @@ template <typename VT>
 int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, const void* inv_diag, int dfmt,
                     Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s) {
     if (!W.rslots.p) {
-        M4_TRY(W.rslots.alloc(3 * kSlotGen));
+        M4_TRY(W.rslots.alloc(kSlotGens * kSlotGen));
         M4_TRY(W.rwords.alloc(kResWords));
     }
     ResArgs a{};
@@ -514,7 +514,7 @@ int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, 
     a.steps = steps;
     a.S = ResSync{W.rslots.p, W.rwords.p, plan.grid};
     if (plan.share) {
-        hipLaunchKernelGGL(k_resident_begin, dim3((3 * kSlotGen + 255) / 256), dim3(256), 0, s, a.S);
+        hipLaunchKernelGGL(k_resident_begin, dim3((kSlotGens * kSlotGen + 255) / 256), dim3(256), 0, s, a.S);
         M4_HIP(hipGetLastError());
     }
 #define M4_RES_ROWS(OP, NE)                                                                        \

@@ -18,10 +18,15 @@ constexpr unsigned kResMeet = 5 * 100000;    // rendezvous: 5 ms of the 100 MHz 
 constexpr unsigned kResPolls = 1u << 22;     // polls of a later wait before it gives up
 
 // ------------------------------------------------------------------ waits between workgroups
-// Sums: three generations of slots, each holding a pending pattern until the
-// workgroup's sum of that generation is stored; a workgroup that has passed
-// generation g knows that all have passed g - 1 and resets its slots of it
-// (= generation g + 2's).  Up to kResFlat workgroups every one publishes to
+// Sums: kSlotGens generations of slots, each slot holding a pending pattern
+// until the workgroup's sum of that generation is stored.  A workgroup that has
+// passed generation g knows that all have passed g - 1 and resets its slots of
+// it, which are generation g + 3's.  That reset has to be seen before anyone
+// polls g + 3: whoever polls it has passed g + 2, for which every workgroup has
+// published, and between a workgroup's reset and its publishing of g + 2 lies a
+// res_exchange (one before every even generation), whose wait_memory completes
+// the reset.  With three generations a reset behind an even one met its next
+// reader with no wait between.  Up to kResFlat workgroups every one publishes to
 // eight copies of a slot row (one per blockIdx % 8, so 1/8 of the readers
 // poll the same lines) and sums the row itself; more meet in eight groups
 // first.  Measured per all-reduce: 1.9 us (32 workgroups), 2.0 (64), 2.5
@@ -30,6 +35,7 @@ constexpr int kResFlat = 128;
 constexpr uint64_t kResPending = 0x7ff5c3c3c3c3c3c3ull;   // signalling NaN: no sum ever is
 constexpr int kSlotRow = 2 * kResMaxGrid;                  // two sums per workgroup
 constexpr int kSlotGen = 8 * kSlotRow;                     // eight copies
+constexpr int kSlotGens = 4;                               // a power of two
 // words: rendezvous arrivals and state, abort flag (own 128-byte lines), then one p flag per workgroup
 enum { RW_ARRIVE = 0, RW_STATE = 32, RW_ABORT = 64, RW_FLAG = 96 };
 constexpr int kResWords = RW_FLAG + kResMaxGrid;
@@ -37,7 +43,7 @@ constexpr int kResWords = RW_FLAG + kResMaxGrid;
 __device__ __forceinline__ bool res_pending(double v) { return (uint64_t)__double_as_longlong(v) == kResPending; }
 
 struct ResSync {
-    double* slots;     // 3 * kSlotGen
+    double* slots;     // kSlotGens * kSlotGen
     unsigned* words;   // kResWords
     int grid;
 };
@@ -95,8 +101,8 @@ __device__ __forceinline__ bool res_allsum(const ResSync& S, int gen, VT a, VT b
         b = res_lane(v, 2 * kResNW - 1);
         bool ok = true;
         const int g = blockIdx.x & 7, m = blockIdx.x >> 3;
-        double* now = S.slots + (size_t)(gen % 3) * kSlotGen;
-        double* old = S.slots + (size_t)((gen + 2) % 3) * kSlotGen;
+        double* now = S.slots + (size_t)(gen & (kSlotGens - 1)) * kSlotGen;
+        double* old = S.slots + (size_t)((gen - 1) & (kSlotGens - 1)) * kSlotGen;
         unsigned* ab = S.words + RW_ABORT;
         const double pend = __longlong_as_double((long long)kResPending);
         if (S.grid <= kResFlat) {
