@@ -413,7 +413,10 @@ ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_form
             int inner = 0;
             for (int d = 1; d + 1 < nd; d++) inner = std::max(inner, std::abs(off[d]));
             int lo = std::abs(off[0]), hi = std::abs(off[nd - 1]);
-            if (inner <= kResHalo) {
+            // The first diagonal is read from memory below -halo and the last one above
+            // +halo, both in LDS otherwise: two diagonals far out on the same side
+            // (the nearer one beyond kResHalo) fit neither.
+            if (inner <= kResHalo && off[0] <= kResHalo && off[nd - 1] >= -kResHalo) {
                 // the fewest rows per lane whose workgroups fit the GPU; two at
                 // least (64,000 rows: 7.1 us per iteration on 63 workgroups,
                 // 7.5 on 125), and one workgroup where the system fits it

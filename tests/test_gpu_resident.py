@@ -81,6 +81,25 @@ def test_resident_cg_matches_launch_per_kernel_loop(m, kind, size, pc):
     assert np.array_equal(xa, xc)   # deterministic
 
 
+@pytest.mark.parametrize("offsets", [(-3000, -2000), (2000, 3000), (-3000, -1024), (-1025, 0), (1024, 1025), (0, 2000)])
+def test_resident_cg_two_diagonals(m, offsets):
+    """Both on one side of the main diagonal, in and beyond the LDS halo (1024)."""
+    n = 9001
+    rng = np.random.default_rng(9)
+    row = np.repeat(np.arange(n), 2)
+    col = row + np.tile(offsets, n)
+    keep = (col >= 0) & (col < n)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(row[keep], minlength=n))]).astype(np.int32)
+    A = m.compressed2D(n, n, rp, col[keep].astype(np.int32), rng.uniform(1, 2, int(keep.sum())))
+    b = m.dense_vector(rng.uniform(1, 2, n))
+    # not a system CG solves: two iterations.  All terms of the first p.q are
+    # positive; 1e-12 leaves room for a cancellation of 1e-3 in the second
+    xa, ia = _few(m, A, None, b, 2, False)
+    xb, ib = _few(m, A, None, b, 2, True)
+    assert ia.iterations() == ib.iterations() == 2
+    assert np.linalg.norm(xa - xb) <= 1e-12 * np.linalg.norm(xb)
+
+
 @pytest.mark.parametrize("layout", ["dia", "sym"])
 @pytest.mark.parametrize("kind,size", [("grid2d", (61, 64)), ("grid2d", (7, 1500)), ("diffusion", 33)])
 def test_resident_cg_layouts_and_oracle(m, kind, size, layout):
