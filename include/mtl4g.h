@@ -131,6 +131,26 @@ int mtl4g_get_reduction_order(void);
  * launched and timed beside it.  Process-wide; for one solve at a time. */
 int mtl4g_set_product_timing(int on);
 int mtl4g_product_timing(double* h_total_us, int64_t* h_count);
+/* Diagnostic (no MTL4 counterpart): how this thread's last CG solve with the
+ * identity or diagonal preconditioner ran.  operand 0: launch per kernel;
+ * otherwise its state was kept on the chip (1, 2: up to 5 / 7 diagonals, 3-5:
+ * up to 8 / 16 / 24 entries per lane of any pattern, 6: diagonals, values
+ * streamed), rows_per_lane rows per lane of each of `workgroups` workgroups,
+ * `halo` neighbouring elements of p in LDS, at most `steps` iterations per
+ * launch; launches, the refused ones among them (another kernel held the
+ * compute units) and the iterations launched one by one after a refusal.  The
+ * solve's bits do not depend on refusals. */
+typedef struct {
+    int32_t operand, rows_per_lane, workgroups, halo, steps;
+    int32_t launches, refused, single_steps;
+} mtl4g_cg_chip_info;
+int mtl4g_cg_chip(mtl4g_cg_chip_info* h_info);
+/* For tests (no MTL4 counterpart): launches refuse_first ..
+ * refuse_first + refuse_count - 1 of every such solve are refused as if another
+ * kernel held the compute units, and a wait between workgroups gives up after
+ * `polls` looks (0: the default), which ends the solve with MTL4G_ERR_TIMEOUT.
+ * 0, 0, 0 restores the defaults.  Process-wide. */
+int mtl4g_set_cg_chip_limits(int32_t refuse_first, int32_t refuse_count, int32_t polls);
 
 /* Device storage for dense_vector (vector/dense_vector.hpp:50-269 keeps its
  * elements in a contiguous_memory_block; here the block lives in HBM).

@@ -61,6 +61,11 @@ class ServerParams(C.Structure):
                 ("rtol", C.c_double), ("cap_bytes", C.c_double), ("per_request", C.c_int32)]
 
 
+class CgChipInfo(C.Structure):
+    _fields_ = [(f, C.c_int32) for f in ("operand", "rows_per_lane", "workgroups", "halo", "steps", "launches",
+                                         "refused", "single_steps")]
+
+
 class ServerStats(C.Structure):
     _fields_ = [("wall_s", C.c_double), ("solves", C.c_int64), ("launches", C.c_int32),
                 ("max_inflight", C.c_int32), ("peak_bytes", C.c_double), ("errors", C.c_int32),
@@ -85,6 +90,8 @@ _SIGS = {
     "mtl4g_get_reduction_order": (_INT, []),
     "mtl4g_set_product_timing": (_INT, [_INT]),
     "mtl4g_product_timing": (_INT, [C.POINTER(_D), C.POINTER(C.c_int64)]),
+    "mtl4g_cg_chip": (_INT, [C.POINTER(CgChipInfo)]),
+    "mtl4g_set_cg_chip_limits": (_INT, [_I32, _I32, _I32]),
     "mtl4g_csr_create": (_INT, [_PP, _I32, _I32, _I64, _P, _P, _P, _INT]),
     "mtl4g_csr_destroy": (_INT, [_P]),
     "mtl4g_csr_info": (_INT, [_P, C.POINTER(_I32), C.POINTER(_I32), C.POINTER(_I64)]),

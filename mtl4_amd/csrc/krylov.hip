@@ -189,14 +189,16 @@ struct EpiCgQ {
     }
 };
 
-// q = A*p alone (product timing beside iterations that run on the chip)
+// q = A*p alone: iterations of an on-chip solve in launches of their own, and
+// (always: at any state) product timing beside those that run on the chip
 template <typename VT>
-struct EpiCgTimed {
+struct EpiCgProduct {
     static constexpr int NP = 0;
     struct Pre {};
     VT* q;
-    Ctl* c;
-    __device__ bool skip() const { return false; }
+    const Ctl* c;
+    int always;
+    __device__ bool skip() const { return !always && (c->done != 0 || c->pause != 0 || c->want_ru != 0); }
     __device__ void prepare() {}
     __device__ Pre preload(int) const { return Pre{}; }
     __device__ void operator()(int row, VT s, const Pre&, VT*) const { __builtin_nontemporal_store(s, q + row); }
@@ -1886,16 +1888,20 @@ static int run_typed(const mtl4g_matrix_s* A, const MT* val, const mtl4g_pc_s* P
         // q = A*p, so one iteration runs per launch and the product's kernel is
         // timed beside it on the same p (q is not read)
         const bool timed = sizeof(VT) == 8 && g_timer.on;
-        auto product = [&]() -> int {
+        auto product = [&](int always) -> int {
+            return launch_csr<VT>(A, val, W.vecs.p, EpiCgProduct<VT>{W.vecs.p + A->n, W.ctl.p, always}, (VT*)nullptr,
+                                  nullptr, s);
+        };
+        auto timed_product = [&]() -> int {
             if (!timed) return MTL4G_OK;
             timer_mark(s, true);
-            M4_TRY(launch_csr<VT>(A, val, W.vecs.p, EpiCgTimed<VT>{W.vecs.p + A->n, W.ctl.p}, (VT*)nullptr, nullptr, s));
+            M4_TRY(product(1));
             timer_mark(s, false);
             return MTL4G_OK;
         };
         bool ran = false;
-        M4_TRY(resident_cg<VT>(A, vfmt, dv, f64 ? MTL4G_F64 : MTL4G_F32, W, x, s, timed ? 1 : kResidentSteps, product,
-                               &ran));
+        M4_TRY(resident_cg<VT>(A, vfmt, dv, f64 ? MTL4G_F64 : MTL4G_F32, W, x, s, timed ? 1 : kResidentSteps,
+                               [&]() { return product(0); }, timed_product, &ran));
         if (ran) return MTL4G_OK;
     }
     // Enqueue chunks of iterations and poll the stop flag between chunks.
@@ -2550,8 +2556,12 @@ static int mixed_typed(mtl4g_matrix_s* A, const MT* val32, const mtl4g_pc_s* P, 
     M4_TRY(refresh());   // initial FP64 residual (Ctl::init set)
     if (pcm != PCM_GENERAL) {
         bool ran = false;
+        auto product = [&]() -> int {
+            return launch_csr<float>(A, val32, W.vecs.p, EpiCgProduct<float>{W.vecs.p + n, W.ctl.p, 0},
+                                     (float*)nullptr, nullptr, s);
+        };
         M4_TRY(resident_cg<float>(A, sizeof(MT) == 4 ? MTL4G_F32 : MTL4G_BF16, d, MTL4G_F32, W, x32, s, kResidentSteps,
-                                  refresh, &ran));
+                                  product, refresh, &ran));
         if (ran) return MTL4G_OK;
     }
     int32_t launched = 0, chunk = 2;

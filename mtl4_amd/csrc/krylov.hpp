@@ -22,7 +22,7 @@ struct Ctl {
     int32_t mixed, pause, want_ru, ru_count, limit, init, restart;
     int32_t stall;           // consecutive FP64 refreshes that did not halve the residual
     int32_t drop;            // the FP32 recurrence went non-finite: discard its correction
-    int32_t refused;         // resident launches in a row that did not get onto the chip
+    int32_t refused;         // resident launches of this solve that did not get onto the chip
     unsigned ticket[4];
 };
 

@@ -18,15 +18,17 @@
 // Workgroups wait for each other (resident_dev.hpp), so all of them must be on the
 // chip at once.  A launch first meets at a rendezvous with a bounded wait:
 // when the grid does not get onto the chip (another kernel holds its CUs) the
-// launch gives up before it has changed anything and the host tries again.
-// After the rendezvous every workgroup is running and every later wait ends;
-// those waits are bounded too and raise an abort flag.
+// launch gives up before it has changed anything, and iterations in launches of
+// their own (k_cg_step) go on from the same state with the same bits until the
+// host tries again.  After the rendezvous every workgroup is running and every
+// later wait ends; those waits are bounded too and raise an abort flag.
 //
 // Ordering: the inter-workgroup protocol of internal.hpp (agent-scope stores
 // and loads; wait_memory before the store that announces).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <map>
 #include <mutex>
@@ -332,7 +334,7 @@ __global__ __launch_bounds__(kResBS) void k_cg_resident(ResArgs a) {
         }
         ok = res_allsum<VT, ONE>(a.S, gen++, s0, s1, sh, L.rr, L.rz);
         if (!ok) break;
-        if (L.head(a.hist) || (int)step >= a.steps) break;
+        if (L.head(a.hist, blockIdx.x == 0 && t == 0) || (int)step >= a.steps) break;
     }
 #pragma unroll
     for (int k = 0; k < R; k++) {
@@ -346,19 +348,128 @@ __global__ __launch_bounds__(kResBS) void k_cg_resident(ResArgs a) {
     if (blockIdx.x == 0 && t == 0) L.leave(a.c, ok);
 }
 
-// Slots pending, words zero, before each launch.
-__global__ void k_resident_begin(ResSync S) {
+// Slots pending, words zero, before each launch; state: RS_OPEN, or RS_REFUSED
+// for a launch that is to be turned away (mtl4g_set_cg_chip_limits).
+__global__ void k_resident_begin(ResSync S, unsigned state) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < kSlotGens * kSlotGen) S.slots[i] = __longlong_as_double((long long)kResPending);
-    if (i < kResWords) S.words[i] = 0u;
+    if (i < kResWords) S.words[i] = i == RW_STATE ? state : 0u;
+}
+
+// ------------------------------------------------------------------ iterations in launches of their own
+// The same state, the same arithmetic per element and every sum in the order of
+// the kernels above: a lane adds up its rows of the plan (`groups` of them, `per`
+// consecutive rows each), then res_allsum's order over lanes, waves and
+// workgroups.  No workgroup waits for another.  p is written first, then the
+// caller's product forms q.
+template <typename VT>
+__global__ __launch_bounds__(kResBS) void k_cg_step_p(ResArgs a) {
+    const Ctl* c = a.c;
+    if (c->done || c->pause || c->want_ru) return;
+    const bool first = c->first != 0;
+    const VT beta = static_cast<VT>(c->beta);
+    const VT* r = static_cast<const VT*>(a.r);
+    VT* p = static_cast<VT*>(a.p);
+    const int64_t stride = (int64_t)gridDim.x * kResBS;
+    for (int64_t i = blockIdx.x * (int64_t)kResBS + threadIdx.x; i < a.n; i += stride) {
+        const VT z = a.d ? res_value<VT>(a.d, a.dfmt, i) * r[i] : r[i];
+        p[i] = first ? z : z + beta * p[i];
+    }
+}
+
+// UPDATE: x, r, the loop head; otherwise p.q and alpha
+template <typename VT, bool UPDATE>
+__global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int groups, int per) {
+    Ctl* c = a.c;
+    if (c->done || c->pause || c->want_ru) return;
+    __shared__ VT part[2 * kResNW];
+    const int t = (int)threadIdx.x, l = t & (kWave - 1), w = t / kWave, G = a.S.grid;
+    int lb = (int)blockIdx.x;
+    if (G % kXcd == 0) lb = xcd_logical_block(lb, G / kXcd);
+    VT* x = static_cast<VT*>(a.x);
+    VT* r = static_cast<VT*>(a.r);
+    const VT* p = static_cast<const VT*>(a.p);
+    const VT alpha = static_cast<VT>(c->alpha);
+    VT s0 = VT(0), s1 = VT(0);
+    for (int k = 0; k < groups; k++)
+        for (int v = 0; v < per; v++) {
+            const int64_t i = ((int64_t)(lb * groups + k) * kResBS + t) * per + v;
+            if (i >= a.n) continue;
+            if (UPDATE) {
+                x[i] = x[i] + alpha * p[i];
+                const VT ri = r[i] - alpha * q[i];
+                r[i] = ri;
+                s0 += ri * ri;
+                s1 += ri * (a.d ? res_value<VT>(a.d, a.dfmt, i) * ri : ri);
+            } else {
+                s0 += p[i] * q[i];
+            }
+        }
+    s0 = res_wave(s0);
+    s1 = res_wave(s1);
+    if (l == 0) {
+        part[w] = s0;
+        part[kResNW + w] = s1;
+    }
+    __syncthreads();
+    if (w == 0) {
+        const VT v = res_row8(l < 2 * kResNW ? part[l] : VT(0));
+        s0 = res_lane(v, kResNW - 1);
+        s1 = res_lane(v, 2 * kResNW - 1);
+        if (l == 0) {
+            st_agent(a.S.slots + 2 * blockIdx.x, (double)s0);
+            st_agent(a.S.slots + 2 * blockIdx.x + 1, (double)s1);
+        }
+    }
+    if (!arrive_last<kResBS>(a.S.words + RW_TICKET, (unsigned)G) || w != 0) return;
+    auto sum = [&](int i, VT& ta, VT& tb) {   // workgroup i's sums
+        ta += (VT)ld_agent(a.S.slots + 2 * i);
+        tb += (VT)ld_agent(a.S.slots + 2 * i + 1);
+    };
+    s0 = s1 = VT(0);
+    if (G <= kResFlat) {
+        for (int i = l; i < G; i += kWave) sum(i, s0, s1);
+    } else {
+        for (int g = 0; g < 8; g++) {
+            VT ga = VT(0), gb = VT(0);
+            if (l < (G - g + 7) / 8) sum(g + 8 * l, ga, gb);
+            ga = res_wave(ga);
+            gb = res_wave(gb);
+            if (l == g) {
+                s0 = ga;
+                s1 = gb;
+            }
+        }
+    }
+    s0 = res_wave(s0);
+    s1 = res_wave(s1);
+    if (l != 0) return;
+    ResLoop<VT> L;
+    L.init(c);
+    if (UPDATE) {
+        L.rr = s0;
+        L.rz = s1;
+        L.head(a.hist, true);
+        L.leave(c, true);
+    } else {
+        L.pq = s0;
+        L.direction();
+        c->alpha = (double)L.alpha;
+        c->alpha_1 = (double)L.pq;
+        c->rho_1 = (double)L.rho_1;
+    }
 }
 
 // ------------------------------------------------------------------ host
 namespace {
 struct Units {
+    struct Device {
+        int used = 0;                        // CUs held by resident grids
+        uint64_t arrived = 0, served = 0;    // claims, in order
+    };
     std::mutex mu;
     std::condition_variable cv;
-    std::map<int, int> used;   // device -> CUs held by resident grids
+    std::map<int, Device> devices;
 };
 Units& units() {
     static Units u;
@@ -370,8 +481,13 @@ ResidentClaim::ResidentClaim(int dev, int n, int total) : device(dev), units(std
     if (!units) return;
     Units& u = mtl4g::units();
     std::unique_lock<std::mutex> lk(u.mu);
-    u.cv.wait(lk, [&] { return u.used[device] + units <= total; });
-    u.used[device] += units;
+    Units::Device& d = u.devices[device];
+    const uint64_t turn = d.arrived++;
+    u.cv.wait(lk, [&] { return d.served == turn && d.used + units <= total; });
+    d.used += units;
+    d.served++;
+    lk.unlock();
+    u.cv.notify_all();
 }
 
 ResidentClaim::~ResidentClaim() {
@@ -379,7 +495,7 @@ ResidentClaim::~ResidentClaim() {
     Units& u = mtl4g::units();
     {
         std::lock_guard<std::mutex> lk(u.mu);
-        u.used[device] -= units;
+        u.devices[device].used -= units;
     }
     u.cv.notify_all();
 }
@@ -478,6 +594,53 @@ ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_form
     return P;
 }
 
+mtl4g_cg_chip_info& resident_info() {
+    static thread_local mtl4g_cg_chip_info info{};
+    return info;
+}
+
+namespace {
+// mtl4g_set_cg_chip_limits
+std::atomic<int32_t> g_refuse_first{0}, g_refuse_count{0}, g_polls{0};
+}  // namespace
+
+// vectors, scalars and waits; the matrix is the launch's own
+template <typename VT>
+static ResArgs resident_args(const ResidentPlan& plan, const mtl4g_matrix_s* A, const void* inv_diag, int dfmt,
+                             Workspace<VT>& W, VT* x) {
+    ResArgs a{};
+    a.n = A->n;
+    a.x = x;
+    a.p = W.vecs.p;
+    a.r = W.vecs.p + 2 * (size_t)A->n;
+    a.d = inv_diag;
+    a.dfmt = dfmt;
+    a.c = W.ctl.p;
+    a.hist = W.hist.p;
+    const int32_t polls = g_polls.load();
+    a.S = ResSync{W.rslots.p, W.rwords.p, plan.grid, polls > 0 ? (unsigned)polls : kResPolls};
+    return a;
+}
+
+template <typename VT>
+int resident_step(int part, const ResidentPlan& plan, const mtl4g_matrix_s* A, const void* inv_diag, int dfmt,
+                  Workspace<VT>& W, VT* x, hipStream_t s) {
+    const ResArgs a = resident_args(plan, A, inv_diag, dfmt, W, x);
+    const VT* q = W.vecs.p + (size_t)A->n;
+    const int groups = plan.groups ? plan.groups : 1 << plan.rows_log2;
+    const int per = plan.groups ? 16 / (int)sizeof(VT) : 1;
+    if (part == RSTEP_P) {
+        const int grid = std::min((A->n + kResBS - 1) / kResBS, 2048);
+        hipLaunchKernelGGL(k_cg_step_p<VT>, dim3(grid), dim3(kResBS), 0, s, a);
+    } else if (part == RSTEP_ALPHA) {
+        hipLaunchKernelGGL((k_cg_step<VT, false>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+    } else {
+        hipLaunchKernelGGL((k_cg_step<VT, true>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+    }
+    M4_HIP(hipGetLastError());
+    return MTL4G_OK;
+}
+
 template <typename VT>
 int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, const void* inv_diag, int dfmt,
                     Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s) {
@@ -485,8 +648,7 @@ int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, 
         M4_TRY(W.rslots.alloc(kSlotGens * kSlotGen));
         M4_TRY(W.rwords.alloc(kResWords));
     }
-    ResArgs a{};
-    a.n = A->n;
+    ResArgs a = resident_args(plan, A, inv_diag, dfmt, W, x);
     const bool sym = A->kernel == MTL4G_SPMV_DIA_SYM;
     if (plan.op == ROP_DIA5 || plan.op == ROP_DIA7 || plan.op == ROP_LARGE) {
         a.doff = sym ? A->dsym_off.p : A->dia_off.p;
@@ -507,17 +669,12 @@ int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, 
     a.fmt = fmt;
     a.halo = plan.halo;
     a.neigh = plan.neigh;
-    a.x = x;
-    a.p = W.vecs.p;
-    a.r = W.vecs.p + 2 * (size_t)A->n;
-    a.d = inv_diag;
-    a.dfmt = dfmt;
-    a.c = W.ctl.p;
-    a.hist = W.hist.p;
     a.steps = steps;
-    a.S = ResSync{W.rslots.p, W.rwords.p, plan.grid};
+    const int32_t nth = resident_info().launches++;
     if (plan.share) {
-        hipLaunchKernelGGL(k_resident_begin, dim3((kSlotGens * kSlotGen + 255) / 256), dim3(256), 0, s, a.S);
+        const int32_t first = g_refuse_first.load();
+        const unsigned state = nth >= first && nth - first < g_refuse_count.load() ? RS_REFUSED : RS_OPEN;
+        hipLaunchKernelGGL(k_resident_begin, dim3((kSlotGens * kSlotGen + 255) / 256), dim3(256), 0, s, a.S, state);
         M4_HIP(hipGetLastError());
     }
 #define M4_RES_ROWS(OP, NE)                                                                        \
@@ -542,9 +699,36 @@ int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, 
     return MTL4G_ERR_INVALID;
 }
 
+template int resident_step<double>(int, const ResidentPlan&, const mtl4g_matrix_s*, const void*, int,
+                                   Workspace<double>&, double*, hipStream_t);
+template int resident_step<float>(int, const ResidentPlan&, const mtl4g_matrix_s*, const void*, int,
+                                  Workspace<float>&, float*, hipStream_t);
 template int resident_launch<double>(const ResidentPlan&, const mtl4g_matrix_s*, int, const void*, int,
                                      Workspace<double>&, double*, int32_t, hipStream_t);
 template int resident_launch<float>(const ResidentPlan&, const mtl4g_matrix_s*, int, const void*, int,
                                     Workspace<float>&, float*, int32_t, hipStream_t);
 
 }  // namespace mtl4g
+
+using namespace mtl4g;
+
+extern "C" {
+
+int mtl4g_cg_chip(mtl4g_cg_chip_info* h_info) {
+    if (!h_info) return MTL4G_ERR_INVALID;
+    *h_info = resident_info();
+    return MTL4G_OK;
+}
+
+int mtl4g_set_cg_chip_limits(int32_t refuse_first, int32_t refuse_count, int32_t polls) {
+    if (refuse_first < 0 || refuse_count < 0 || polls < 0) {
+        set_error("mtl4g_set_cg_chip_limits: arguments must not be negative");
+        return MTL4G_ERR_INVALID;
+    }
+    g_refuse_first.store(refuse_first);
+    g_refuse_count.store(refuse_count);
+    g_polls.store(polls);
+    return MTL4G_OK;
+}
+
+}  // extern "C"

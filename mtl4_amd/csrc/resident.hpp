@@ -1,6 +1,8 @@
 // resident.hpp -- itl::cg with its state on the chip (resident.hip, resident_large.hip).
 #pragma once
 
+#include <algorithm>
+
 #include "krylov.hpp"
 
 namespace mtl4g {
@@ -8,15 +10,21 @@ namespace mtl4g {
 // Runs CG iterations from the state the loop head left in W (r, p, Ctl;
 // cg.hpp:94-108), the identity or diagonal preconditioner, inside one kernel
 // per batch of iterations.  Returns MTL4G_OK with *ran = true when the solve
-// stopped (Ctl::done set), or with *ran = false when this path does not take
-// the matrix (or the GPU stayed too busy to hold the whole grid): the caller's
-// own loop goes on from the same state.  inv_diag: n values of the vector
-// type's precision or of the other one (dfmt MTL4G_F64 / MTL4G_F32), null for
-// the identity.  A launch runs at most `steps` iterations; after() is enqueued
+// stopped (Ctl::done set), or with *ran = false, and nothing done, when this
+// path does not take the matrix.  inv_diag: n values of the vector type's
+// precision or of the other one (dfmt MTL4G_F64 / MTL4G_F32), null for the
+// identity.  A launch runs at most `steps` iterations; after() is enqueued
 // behind each (mixed precision: the FP64 refresh).
-template <typename VT, typename After>
+//
+// A launch that does not get onto the chip (another stream's or process's
+// kernel holds compute units) is followed by iterations in launches of their
+// own, which need no more than one compute unit at a time and form every sum in
+// the same order: the solve goes on, with the same bits.  product() enqueues
+// q = A*p for those (p, q: the first two vectors of W).  The chip is tried
+// again after kStepsMin of them, and after twice as many each time it refuses.
+template <typename VT, typename Product, typename After>
 int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag, int dfmt, Workspace<VT>& W, VT* x,
-                hipStream_t s, int32_t steps, After after, bool* ran);
+                hipStream_t s, int32_t steps, Product product, After after, bool* ran);
 
 // The pieces the template above is made of.
 struct ResidentPlan {
@@ -33,11 +41,19 @@ ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_form
 template <typename VT>
 int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
                     int dfmt, Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s);
+// The three parts of an iteration around q = A*p and behind it, each a launch.
+enum { RSTEP_P = 0, RSTEP_ALPHA = 1, RSTEP_UPDATE = 2 };
+template <typename VT>
+int resident_step(int part, const ResidentPlan& plan, const mtl4g_matrix_s* A, const void* inv_diag, int dfmt,
+                  Workspace<VT>& W, VT* x, hipStream_t s);
+// What the last solve of this thread did here (mtl4g_cg_chip).
+mtl4g_cg_chip_info& resident_info();
 
 // Compute units taken by resident grids of this process, per device: a grid
 // that spans several workgroups takes its CUs before it is launched and gives
 // them back after it has finished, so two such grids never wait for each
-// other's CUs.
+// other's CUs.  Served in the order of arrival: a solve that gives its units
+// back and asks again at once stands behind those that waited.
 struct ResidentClaim {
     int device, units;
     ResidentClaim(int device, int units, int total);
@@ -49,35 +65,61 @@ struct ResidentClaim {
 // iterations per launch: a few milliseconds, so that other streams' kernels
 // wait no longer for the compute units
 constexpr int32_t kResidentSteps = 256;
-constexpr int kResidentRefusals = 2000;      // refused launches before the caller's loop takes over
+// Iterations in launches of their own after a refusal: at first about as long
+// as the millisecond the refusal took; doubled, so that a GPU that stays shared
+// costs a solve little more than those launches.
+constexpr int kStepsMin = 32, kStepsMax = 512;
+constexpr int kStepsPerRefresh = 4;   // a pause for after() skips at most three of them
 
-template <typename VT, typename After>
+template <typename VT, typename Product, typename After>
 int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag, int dfmt, Workspace<VT>& W, VT* x,
-                hipStream_t s, int32_t steps, After after, bool* ran) {
+                hipStream_t s, int32_t steps, Product product, After after, bool* ran) {
     *ran = false;
+    mtl4g_cg_chip_info& info = resident_info();
+    info = mtl4g_cg_chip_info{};
     if (W.shared_gpu) return MTL4G_OK;
     const ResidentPlan plan = resident_plan(
         A, (int)sizeof(VT), value_format, !inv_diag || dfmt == (sizeof(VT) == 8 ? MTL4G_F64 : MTL4G_F32));
     if (!plan.op) return MTL4G_OK;
-    int launches = 1;
+    info.operand = plan.op;
+    info.workgroups = plan.grid;
+    info.rows_per_lane = plan.groups ? plan.groups * 16 / (int)sizeof(VT) : 1 << plan.rows_log2;
+    info.halo = plan.halo;
+    info.steps = steps;
+    auto poll = [&]() -> int {
+        M4_HIP(hipMemcpyAsync(W.h_ctl, W.ctl.p, sizeof(Ctl), hipMemcpyDeviceToHost, s));
+        M4_HIP(hipStreamSynchronize(s));
+        return MTL4G_OK;
+    };
+    int launches = 1, chunk = kStepsMin;
     for (;;) {
-        int32_t refused = 0;
         {
             ResidentClaim claim(A->device, plan.grid > 1 ? plan.grid : 0, A->cus);
             for (int k = 0; k < launches; k++) {
                 M4_TRY(resident_launch<VT>(plan, A, value_format, inv_diag, dfmt, W, x, steps, s));
                 M4_TRY(after());
             }
-            M4_HIP(hipMemcpyAsync(W.h_ctl, W.ctl.p, sizeof(Ctl), hipMemcpyDeviceToHost, s));
-            M4_HIP(hipStreamSynchronize(s));
-            refused = W.h_ctl->refused;
+            M4_TRY(poll());
+        }
+        const bool refused = W.h_ctl->refused != info.refused;
+        info.refused = W.h_ctl->refused;
+        if (!W.h_ctl->done && refused) {
+            for (int k = 0; k < chunk; k++) {
+                M4_TRY(resident_step<VT>(RSTEP_P, plan, A, inv_diag, dfmt, W, x, s));
+                M4_TRY(product());
+                M4_TRY(resident_step<VT>(RSTEP_ALPHA, plan, A, inv_diag, dfmt, W, x, s));
+                M4_TRY(resident_step<VT>(RSTEP_UPDATE, plan, A, inv_diag, dfmt, W, x, s));
+                if (k % kStepsPerRefresh == kStepsPerRefresh - 1) M4_TRY(after());
+            }
+            info.single_steps += chunk;
+            M4_TRY(poll());
         }
         if (W.h_ctl->done) {
             *ran = true;
             return MTL4G_OK;
         }
-        if (refused > kResidentRefusals) return MTL4G_OK;
-        launches = 4;
+        chunk = refused ? std::min(2 * chunk, kStepsMax) : kStepsMin;
+        launches = refused ? 1 : 4;
     }
 }
 

@@ -14,7 +14,7 @@ namespace mtl4g {
 constexpr int kResBS = 512;                  // 8 waves per workgroup, 256 registers per lane
 constexpr int kResMaxGrid = 256;             // one workgroup per CU
 constexpr int kResHalo = 1024;               // diagonals this close are read from LDS, others from memory
-constexpr unsigned kResMeet = 5 * 100000;    // rendezvous: 5 ms of the 100 MHz clock
+constexpr unsigned kResMeet = 100000;        // rendezvous: 1 ms of the 100 MHz clock
 constexpr unsigned kResPolls = 1u << 22;     // polls of a later wait before it gives up
 
 // ------------------------------------------------------------------ waits between workgroups
@@ -36,8 +36,10 @@ constexpr uint64_t kResPending = 0x7ff5c3c3c3c3c3c3ull;   // signalling NaN: no 
 constexpr int kSlotRow = 2 * kResMaxGrid;                  // two sums per workgroup
 constexpr int kSlotGen = 8 * kSlotRow;                     // eight copies
 constexpr int kSlotGens = 4;                               // a power of two
-// words: rendezvous arrivals and state, abort flag (own 128-byte lines), then one p flag per workgroup
-enum { RW_ARRIVE = 0, RW_STATE = 32, RW_ABORT = 64, RW_FLAG = 96 };
+// words: rendezvous arrivals and state, abort flag, ticket of the single steps (own
+// 128-byte lines), then one p flag per workgroup
+enum { RW_ARRIVE = 0, RW_STATE = 32, RW_ABORT = 64, RW_TICKET = 96, RW_FLAG = 128 };
+enum { RS_OPEN = 0, RS_MET = 1, RS_REFUSED = 2 };   // rendezvous state
 constexpr int kResWords = RW_FLAG + kResMaxGrid;
 
 __device__ __forceinline__ bool res_pending(double v) { return (uint64_t)__double_as_longlong(v) == kResPending; }
@@ -46,18 +48,19 @@ struct ResSync {
     double* slots;     // kSlotGens * kSlotGen
     unsigned* words;   // kResWords
     int grid;
+    unsigned polls;    // kResPolls
 };
 
 // Two neighbouring values polled until both are there; false when the wait
 // expired or another workgroup has given up.
-__device__ __forceinline__ bool res_poll2(const double* p, unsigned* abort, double& a, double& b) {
+__device__ __forceinline__ bool res_poll2(const double* p, unsigned* abort, unsigned polls, double& a, double& b) {
     a = ld_agent(p);
     b = ld_agent(p + 1);
     unsigned it = 0;
 #pragma clang loop unroll(disable)
     while (res_pending(a) || res_pending(b)) {
         if ((++it & 255u) == 0 && ld_agent(abort) != 0u) return false;
-        if (it > kResPolls) {
+        if (it > polls) {
             st_agent(abort, 1u);
             return false;
         }
@@ -115,7 +118,7 @@ __device__ __forceinline__ bool res_allsum(const ResSync& S, int gen, VT a, VT b
 #pragma clang loop unroll(disable)
             for (int i = l; i < S.grid; i += kWave) {
                 double va = 0, vb = 0;
-                ok = res_poll2(row + 2 * i, ab, va, vb) && ok;
+                ok = res_poll2(row + 2 * i, ab, S.polls, va, vb) && ok;
                 a += (VT)va;
                 b += (VT)vb;
             }
@@ -137,7 +140,7 @@ __device__ __forceinline__ bool res_allsum(const ResSync& S, int gen, VT a, VT b
             }
             if (m == 0) {
                 double va = 0, vb = 0;
-                if (l < gs) ok = res_poll2(grp + 2 * l, ab, va, vb);
+                if (l < gs) ok = res_poll2(grp + 2 * l, ab, S.polls, va, vb);
                 a = res_wave((VT)va);
                 b = res_wave((VT)vb);
                 if (l < 8) {
@@ -146,7 +149,7 @@ __device__ __forceinline__ bool res_allsum(const ResSync& S, int gen, VT a, VT b
                 }
             }
             double va = 0, vb = 0;
-            if (l < 8) ok = res_poll2(top + 2 * l, ab, va, vb) && ok;
+            if (l < 8) ok = res_poll2(top + 2 * l, ab, S.polls, va, vb) && ok;
             a = res_wave((VT)va);
             b = res_wave((VT)vb);
             if (l == 0) {
@@ -179,21 +182,21 @@ __device__ __forceinline__ bool res_meet(const ResSync& S, int* sh) {
         unsigned* st = S.words + RW_STATE;
         const unsigned before =
             __hip_atomic_fetch_add(S.words + RW_ARRIVE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned expect = 0u;
+        unsigned expect = RS_OPEN;
         if (before + 1u == (unsigned)S.grid)
-            __hip_atomic_compare_exchange_strong(st, &expect, 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+            __hip_atomic_compare_exchange_strong(st, &expect, (unsigned)RS_MET, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
         const uint64_t t0 = wall_clock64();
         unsigned v;
-        while ((v = ld_agent(st)) == 0u) {
+        while ((v = ld_agent(st)) == RS_OPEN) {
             if (wall_clock64() - t0 > kResMeet) {
-                expect = 0u;
-                __hip_atomic_compare_exchange_strong(st, &expect, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT);
+                expect = RS_OPEN;
+                __hip_atomic_compare_exchange_strong(st, &expect, (unsigned)RS_REFUSED, __ATOMIC_RELAXED,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __builtin_amdgcn_s_sleep(1);
         }
-        *sh = v == 1u;
+        *sh = v == RS_MET;
     }
     __syncthreads();
     return __builtin_amdgcn_readfirstlane(*sh) != 0;
@@ -217,7 +220,7 @@ __device__ __forceinline__ bool res_exchange(const ResSync& S, int lb, int neigh
 #pragma clang loop unroll(disable)
             while (ld_agent(S.words + RW_FLAG + i) < step) {
                 if ((++it & 255u) == 0 && ld_agent(ab) != 0u) { ok = false; break; }
-                if (it > kResPolls) {
+                if (it > S.polls) {
                     st_agent(ab, 1u);
                     ok = false;
                     break;
@@ -266,7 +269,9 @@ struct ResLoop {
         rho = static_cast<VT>(c->rho);
         rho_1 = static_cast<VT>(c->rho_1);
         beta = static_cast<VT>(c->beta);
-        alpha = pq = rr = rz = VT(0);
+        alpha = static_cast<VT>(c->alpha);
+        pq = static_cast<VT>(c->alpha_1);
+        rr = rz = VT(0);
         norm_r0 = c->norm_r0;
         atol = c->atol;
         // conv_test: resid <= rtol*norm_r0 || resid <= atol (norm_r0 == 0: atol alone)
@@ -286,12 +291,13 @@ struct ResLoop {
         rho_1 = rho;
     }
     // iter_finished / mixed_check (krylov_dev.hpp) on rr and, when the loop
-    // goes on, the next rho and beta  (cg.hpp:94-101); true: leave the kernel
-    __device__ __forceinline__ bool head(double* hist) {
+    // goes on, the next rho and beta  (cg.hpp:94-101); true: leave the kernel.
+    // writer: the one lane of the grid that records the residual
+    __device__ __forceinline__ bool head(double* hist, bool writer) {
         resid = (double)std::sqrt(std::fabs(rr));
         const bool conv = resid <= stop, out = i >= max_iter, bad = !isfinite(resid);
         if (!mixed) {
-            if (blockIdx.x == 0 && threadIdx.x == 0 && hist_n < hist_cap) hist[hist_n] = resid;
+            if (writer && hist_n < hist_cap) hist[hist_n] = resid;
             hist_n++;
             done = conv || out || bad;
             if (done && !conv) {
@@ -313,7 +319,6 @@ struct ResLoop {
         return done || want_ru;
     }
     __device__ __forceinline__ void leave(Ctl* c, bool ok) const {
-        c->refused = 0;
         if (!mixed) c->resid = resid;
         c->rr = (double)rr;
         c->alpha = (double)alpha;

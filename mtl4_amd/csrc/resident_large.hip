@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kResBS) void k_cg_large(ResArgs a) {
         }
         ok = res_allsum<VT, false>(a.S, gen++, s0, s1, sh, L.rr, L.rz);
         if (!ok) break;
-        if (L.head(a.hist) || (int)step >= a.steps) break;
+        if (L.head(a.hist, blockIdx.x == 0 && t == 0) || (int)step >= a.steps) break;
     }
 #pragma unroll
     for (int k = 0; k < K; k++) {

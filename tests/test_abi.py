@@ -80,3 +80,16 @@ def test_product_timing_arguments():
     assert lib.mtl4g_set_product_timing(2) == _lib.ERR_INVALID
     assert lib.mtl4g_product_timing(None, None) == _lib.ERR_INVALID
     assert lib.mtl4g_set_product_timing(0) == 0
+
+
+def test_cg_chip_arguments():
+    """The diagnostic of the on-chip CG checks its arguments on the host."""
+    import ctypes as C
+    from mtl4_amd import _lib
+    lib = _lib.lib()
+    assert lib.mtl4g_cg_chip(None) == _lib.ERR_INVALID
+    info = _lib.CgChipInfo()
+    assert lib.mtl4g_cg_chip(C.byref(info)) == 0 and info.operand == info.launches == 0
+    for bad in ((-1, 0, 0), (0, -1, 0), (0, 0, -1)):
+        assert lib.mtl4g_set_cg_chip_limits(*bad) == _lib.ERR_INVALID
+    assert lib.mtl4g_set_cg_chip_limits(0, 0, 0) == 0
