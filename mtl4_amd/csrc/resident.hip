@@ -669,7 +669,10 @@ int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int fmt, 
     a.fmt = fmt;
     a.halo = plan.halo;
     a.neigh = plan.neigh;
-    a.steps = steps;
+    if (plan.op == ROP_LARGE)
+        steps = std::min(steps, (int32_t)std::max<int64_t>(
+                                    1, kResidentSteps * kResidentVector / ((int64_t)A->n * (int64_t)sizeof(VT))));
+    a.steps = resident_info().steps = steps;
     const int32_t nth = resident_info().launches++;
     if (plan.share) {
         const int32_t first = g_refuse_first.load();

@@ -62,9 +62,13 @@ struct ResidentClaim {
     ResidentClaim& operator=(const ResidentClaim&) = delete;
 };
 
-// iterations per launch: a few milliseconds, so that other streams' kernels
-// wait no longer for the compute units
+// Iterations per launch, so that other streams' kernels wait no more than about
+// 5 ms for the compute units: 256 of up to 20 us while the matrix is in
+// registers; streamed ones take time by their rows (102^3 15.5 us, 160^3 73 us in
+// FP64), so vectors of more than 8 MB get as many fewer (160^3: 65, 4.7 ms; one
+// launch of 256 held all compute units for 18.8 ms).
 constexpr int32_t kResidentSteps = 256;
+constexpr int64_t kResidentVector = 8 << 20;
 // Iterations in launches of their own after a refusal: at first about as long
 // as the millisecond the refusal took; doubled, so that a GPU that stays shared
 // costs a solve little more than those launches.

@@ -299,9 +299,7 @@ __global__ __launch_bounds__(kResBS) void k_cg_large(ResArgs a) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(res_u4, xk[KEEP ? k : 0]), bx,
                                                    row_at + k * (STEP * VB), 0, 0);
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(res_u4, r[k]), br, row_at + k * (STEP * VB), 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(res_u4, *reinterpret_cast<const VV*>(mine + k * STEP)),
-                                               bp, row_at + k * (STEP * VB), 0, 0);
-    }
+    }   // p is in memory since the last exchange
     if (blockIdx.x == 0 && t == 0) L.leave(a.c, ok);
 }
 

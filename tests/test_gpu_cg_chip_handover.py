@@ -177,6 +177,19 @@ def test_solve_beside_a_batch_that_holds_compute_units(m):
     assert not failed and not t.is_alive()
 
 
+@pytest.mark.parametrize("sizes", [(102, 103, 102), (160, 160, 160)])
+def test_a_launch_of_a_large_system_stays_short(m, sizes):
+    """All compute units are held for about 5 ms at most: iterations per launch
+    fall with the rows where these set an iteration's time."""
+    rp, ci, va = _grid(sizes)
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    b = A * m.dense_vector(np.random.default_rng(5).uniform(-1, 1, n))
+    x, h, info = _cg(m, A, m.pc.diagonal(A), b, 300)
+    assert info.operand == 6 and info.steps * n * 8 <= 256 * (8 << 20) < (info.steps + 1) * n * 8
+    assert info.launches >= -(-300 // info.steps) and len(h) == 301 and np.isfinite(h).all()
+
+
 def test_a_waiting_solve_is_served_in_turn(m):
     """Two solves that each need the whole GPU: the one that came later does not
     wait until the other has finished all its iterations."""
