@@ -377,11 +377,13 @@ __global__ __launch_bounds__(kResBS) void k_cg_step_p(ResArgs a) {
     }
 }
 
-// UPDATE: x, r, the loop head; otherwise p.q and alpha
-template <typename VT, bool UPDATE>
+// PART: RSTEP_ALPHA p.q and alpha; RSTEP_UPDATE x, r, the loop head; RSTEP_RESID
+// the residual that the loop head recorded last
+template <typename VT, int PART>
 __global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int groups, int per) {
     Ctl* c = a.c;
-    if (c->done || c->pause || c->want_ru) return;
+    constexpr bool UPDATE = PART == RSTEP_UPDATE;
+    if (PART != RSTEP_RESID && (c->done || c->pause || c->want_ru)) return;
     __shared__ VT part[2 * kResNW];
     const int t = (int)threadIdx.x, l = t & (kWave - 1), w = t / kWave, G = a.S.grid;
     int lb = (int)blockIdx.x;
@@ -401,6 +403,8 @@ __global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int 
                 r[i] = ri;
                 s0 += ri * ri;
                 s1 += ri * (a.d ? res_value<VT>(a.d, a.dfmt, i) * ri : ri);
+            } else if (PART == RSTEP_RESID) {
+                s0 += r[i] * r[i];
             } else {
                 s0 += p[i] * q[i];
             }
@@ -444,6 +448,12 @@ __global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int 
     s0 = res_wave(s0);
     s1 = res_wave(s1);
     if (l != 0) return;
+    if (PART == RSTEP_RESID) {
+        c->rr = (double)s0;
+        c->resid = (double)std::sqrt(std::fabs(s0));
+        if (c->hist_n > 0 && c->hist_n <= c->hist_cap) a.hist[c->hist_n - 1] = c->resid;
+        return;
+    }
     ResLoop<VT> L;
     L.init(c);
     if (UPDATE) {
@@ -633,9 +643,13 @@ int resident_step(int part, const ResidentPlan& plan, const mtl4g_matrix_s* A, c
         const int grid = std::min((A->n + kResBS - 1) / kResBS, 2048);
         hipLaunchKernelGGL(k_cg_step_p<VT>, dim3(grid), dim3(kResBS), 0, s, a);
     } else if (part == RSTEP_ALPHA) {
-        hipLaunchKernelGGL((k_cg_step<VT, false>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_ALPHA>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+    } else if (part == RSTEP_UPDATE) {
+        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_UPDATE>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
     } else {
-        hipLaunchKernelGGL((k_cg_step<VT, true>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+        // a launch of one workgroup has not set the words
+        hipLaunchKernelGGL(k_resident_begin, dim3((kSlotGens * kSlotGen + 255) / 256), dim3(256), 0, s, a.S, RS_OPEN);
+        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_RESID>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
     }
     M4_HIP(hipGetLastError());
     return MTL4G_OK;

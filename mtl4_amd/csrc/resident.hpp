@@ -41,8 +41,9 @@ ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_form
 template <typename VT>
 int resident_launch(const ResidentPlan& plan, const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
                     int dfmt, Workspace<VT>& W, VT* x, int32_t steps, hipStream_t s);
-// The three parts of an iteration around q = A*p and behind it, each a launch.
-enum { RSTEP_P = 0, RSTEP_ALPHA = 1, RSTEP_UPDATE = 2 };
+// The three parts of an iteration around q = A*p and behind it, each a launch;
+// RSTEP_RESID: the residual of a solve that stopped, from the rows alone.
+enum { RSTEP_P = 0, RSTEP_ALPHA = 1, RSTEP_UPDATE = 2, RSTEP_RESID = 3 };
 template <typename VT>
 int resident_step(int part, const ResidentPlan& plan, const mtl4g_matrix_s* A, const void* inv_diag, int dfmt,
                   Workspace<VT>& W, VT* x, hipStream_t s);
@@ -119,6 +120,11 @@ int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
             M4_TRY(poll());
         }
         if (W.h_ctl->done) {
+            // An infinite alpha (p.q = 0) makes NaN of 0 - alpha*0 in the places of the
+            // grid that hold no row, and of the residual with them.  Formed again here:
+            // masking the places in the loop cost 3 % of a 160^3 and a 64^2 solve.
+            if (W.h_ctl->status == MTL4G_ERR_NONFINITE && !W.h_ctl->mixed)
+                M4_TRY(resident_step<VT>(RSTEP_RESID, plan, A, inv_diag, dfmt, W, x, s));
             *ran = true;
             return MTL4G_OK;
         }

@@ -3,6 +3,7 @@ iterations on systems whose rows fit the registers of the GPU's compute units.
 Compared with the launch-per-kernel loop (which runs MTL4's summation order)
 after a few iterations, where only the order of the sums differs, and with the
 oracle at convergence."""
+import io
 import threading
 
 import numpy as np
@@ -128,7 +129,6 @@ def test_resident_cg_history_start_vector_and_limits(m):
     rng = np.random.default_rng(7)
     x0 = rng.uniform(-1, 1, n)
     b = m.dense_vector(rng.uniform(-1, 1, n))
-    import io
     out = io.StringIO()
     it = m.cyclic_iteration(b, 400, 1e-10, 0.0, 1, out)
     x = m.dense_vector(x0)
@@ -157,6 +157,40 @@ def test_resident_cg_nonfinite(m):
     bd, x = m.dense_vector(b), m.dense_vector(n)
     with pytest.raises(m.nonfinite_error):
         m.cg(A, x, bd, m.pc.diagonal(A), m.basic_iteration(1.0, 50, 1e-10))
+
+
+def _indefinite(kind):
+    """p.q = 0 for p = (1, 1, ..), q nowhere 0, on a size that leaves places without rows."""
+    import scipy.sparse as sp
+    if kind == "csr":       # one diagonal: the operand for any pattern
+        n = 1002
+        A = sp.diags(np.tile([1.0, -1.0], n // 2), format="csr")
+    elif kind.startswith("dia"):     # [[0, 1], [-1, 0]] blocks; one: a single workgroup
+        n = 902 if kind == "dia_one" else 9002
+        up = np.tile([1.0, 0.0], n // 2)[:-1]
+        A = sp.diags([-up, up], [-1, 1], format="csr")
+        A.eliminate_zeros()
+    else:                   # five diagonals, more rows than the registers hold
+        n = 1050002
+        z = np.zeros(n)
+        A = sp.diags([z[7:], z[1:], np.tile([1.0, -1.0], n // 2), z[1:], z[7:]], [-7, -1, 0, 1, 7], format="csr")
+    A.sort_indices()
+    return n, A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data
+
+
+@pytest.mark.parametrize("kind", ["csr", "dia", "dia_one", "large"])
+def test_resident_cg_infinite_step(m, kind):
+    """alpha = rho / 0: the residual reported is the infinite one of the rows."""
+    n, rp, ci, va = _indefinite(kind)
+    A = m.compressed2D(n, n, rp, ci, va)
+    b = m.dense_vector(np.ones(n))
+    got = []
+    for order in (m.ORDER_TREE, m.ORDER_MTL4):
+        it = m.cyclic_iteration(b, 50, 1e-10, 0.0, 1, io.StringIO())
+        with m.reduction_order(order), pytest.raises(m.nonfinite_error):
+            m.cg(A, m.dense_vector(n), b, None, it)
+        got.append((it.iterations(), it.resid(), list(it.history)))
+    assert got[0] == got[1] == (1, np.inf, [np.sqrt(n), np.inf])
 
 
 def test_resident_cg_concurrent_threads(m):
