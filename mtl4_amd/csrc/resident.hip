@@ -575,7 +575,9 @@ ResidentPlan resident_plan(const mtl4g_matrix_s* A, int vt_bytes, int value_form
                     P.op = ROP_LARGE;
                     P.groups = groups;
                     P.grid = (int)((n + rows - 1) / rows);
+                    // whole groups, so that the workgroup's own rows start on 16 bytes of the LDS
                     P.halo = std::max({inner, lo <= kResHalo ? lo : 0, hi <= kResHalo ? hi : 0});
+                    P.halo = (P.halo + per - 1) / per * per;
                     P.neigh = (int)std::min<int64_t>(P.grid, (std::max(lo, hi) + rows - 1) / rows);
                     P.share = true;
                     return P;

@@ -123,7 +123,7 @@ __global__ __launch_bounds__(kResBS) void k_cg_large(ResArgs a) {
         }
     }
     const bool flo = off[0] < -halo, fhi = off[ND - 1] > halo;
-    VT* mine = lds + halo + t * V;
+    VT* mine = lds + halo + t * V;   // on 16 bytes: the halo is whole groups
     VV r[K], q[K];   // q holds z between the update and the next direction
     VV xk[KEEP ? K : 1], dk[KEEP ? K : 1];
     // The lane's places are made opaque at the head of each phase: offsets are

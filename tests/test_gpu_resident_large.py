@@ -117,3 +117,25 @@ def test_large_cg_vectors_off_a_16_byte_boundary(m, sizes):
         xs.append(x.numpy().copy())
         assert float(buf[:shift].abs().sum() + buf[shift + n:].abs().sum()) == 0.0
     assert np.array_equal(xs[0], xs[1])
+
+
+@pytest.mark.parametrize("sizes,mixed", [((1500, 1000), False), ((1001, 1600), False), ((102, 103, 102), False),
+                                         ((1480, 1424), True), ((130, 130, 130), True)])
+def test_large_cg_halo_is_whole_groups(m, sizes, mixed):
+    """The workgroup's rows lie behind the halo in LDS and are read 16 bytes at a
+    time: 2 FP64 or 4 FP32 values."""
+    import ctypes as C
+    rp, ci, va = _grid(sizes)
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    A.set_kernel(m._lib.SPMV_DIA, 4, 4)
+    b = A * m.dense_vector(np.random.default_rng(5).uniform(-1, 1, n))
+    x = m.dense_vector(n)
+    if mixed:
+        m.ir_solve(A, x, b, m.basic_iteration(b, 20000, 1e-10), m.pc.diagonal(A, m.F32))
+    else:
+        m.cg(A, x, b, None, m.basic_iteration(b, 3, 0.0))
+    info = m._lib.CgChipInfo()
+    m._lib.check(m._lib.lib().mtl4g_cg_chip(C.byref(info)))
+    near = max(o for o in (1, sizes[0], n // sizes[-1]) if o <= 1024)
+    assert info.operand == 6 and near <= info.halo < near + 4 and info.halo % (4 if mixed else 2) == 0
