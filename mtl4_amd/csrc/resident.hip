@@ -370,17 +370,28 @@ __global__ __launch_bounds__(kResBS) void k_cg_step_p(ResArgs a) {
     const VT beta = static_cast<VT>(c->beta);
     const VT* r = static_cast<const VT*>(a.r);
     VT* p = static_cast<VT*>(a.p);
+    constexpr int U = 4;   // elements at once
     const int64_t stride = (int64_t)gridDim.x * kResBS;
-    for (int64_t i = blockIdx.x * (int64_t)kResBS + threadIdx.x; i < a.n; i += stride) {
-        const VT z = a.d ? res_value<VT>(a.d, a.dfmt, i) * r[i] : r[i];
-        p[i] = first ? z : z + beta * p[i];
+    for (int64_t i0 = blockIdx.x * (int64_t)kResBS + threadIdx.x; i0 < a.n; i0 += U * stride) {
+        VT z[U], old[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t i = min(i0 + u * stride, (int64_t)a.n - 1);
+            z[u] = a.d ? res_value<VT>(a.d, a.dfmt, i) * r[i] : r[i];
+            old[u] = p[i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * stride < a.n) p[i0 + u * stride] = first ? z[u] : z[u] + beta * old[u];
     }
 }
 
 // PART: RSTEP_ALPHA p.q and alpha; RSTEP_UPDATE x, r, the loop head; RSTEP_RESID
-// the residual that the loop head recorded last
-template <typename VT, int PART>
-__global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int groups, int per) {
+// the residual that the loop head recorded last.
+// Bound by memory at 160^3 (four launches, 623 MB, 145 us per iteration; one row
+// at a time instead of four groups 157), by the launches at 61^3 (28 us).
+template <typename VT, int PART, int PER>
+__global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int groups) {
     Ctl* c = a.c;
     constexpr bool UPDATE = PART == RSTEP_UPDATE;
     if (PART != RSTEP_RESID && (c->done || c->pause || c->want_ru)) return;
@@ -393,22 +404,40 @@ __global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int 
     const VT* p = static_cast<const VT*>(a.p);
     const VT alpha = static_cast<VT>(c->alpha);
     VT s0 = VT(0), s1 = VT(0);
-    for (int k = 0; k < groups; k++)
-        for (int v = 0; v < per; v++) {
-            const int64_t i = ((int64_t)(lb * groups + k) * kResBS + t) * per + v;
-            if (i >= a.n) continue;
+    constexpr int U = 4;   // groups at once
+    for (int k0 = 0; k0 < groups; k0 += U) {
+        VT pi[U * PER], qi[U * PER], ri[U * PER], xi[U * PER], di[U * PER];
+        auto row = [&](int e) {
+            const int64_t i = ((int64_t)(lb * groups + k0 + e / PER) * kResBS + t) * PER + e % PER;
+            return k0 + e / PER < groups && i < a.n ? i : (int64_t)-1;
+        };
+#pragma unroll
+        for (int e = 0; e < U * PER; e++) {
+            const int64_t i = max(row(e), (int64_t)0);
+            if (PART != RSTEP_RESID) pi[e] = p[i], qi[e] = q[i];
+            if (PART != RSTEP_ALPHA) ri[e] = r[i];
             if (UPDATE) {
-                x[i] = x[i] + alpha * p[i];
-                const VT ri = r[i] - alpha * q[i];
-                r[i] = ri;
-                s0 += ri * ri;
-                s1 += ri * (a.d ? res_value<VT>(a.d, a.dfmt, i) * ri : ri);
-            } else if (PART == RSTEP_RESID) {
-                s0 += r[i] * r[i];
-            } else {
-                s0 += p[i] * q[i];
+                xi[e] = x[i];
+                di[e] = a.d ? res_value<VT>(a.d, a.dfmt, i) : VT(1);
             }
         }
+#pragma unroll
+        for (int e = 0; e < U * PER; e++) {
+            const int64_t i = row(e);
+            if (i < 0) continue;
+            if (UPDATE) {
+                x[i] = xi[e] + alpha * pi[e];
+                const VT rn = ri[e] - alpha * qi[e];
+                r[i] = rn;
+                s0 += rn * rn;
+                s1 += rn * (di[e] * rn);
+            } else if (PART == RSTEP_RESID) {
+                s0 += ri[e] * ri[e];
+            } else {
+                s0 += pi[e] * qi[e];
+            }
+        }
+    }
     s0 = res_wave(s0);
     s1 = res_wave(s1);
     if (l == 0) {
@@ -640,18 +669,22 @@ int resident_step(int part, const ResidentPlan& plan, const mtl4g_matrix_s* A, c
     const ResArgs a = resident_args(plan, A, inv_diag, dfmt, W, x);
     const VT* q = W.vecs.p + (size_t)A->n;
     const int groups = plan.groups ? plan.groups : 1 << plan.rows_log2;
-    const int per = plan.groups ? 16 / (int)sizeof(VT) : 1;
+    auto sums = [&](auto one, auto vec) {
+        if (plan.groups) hipLaunchKernelGGL(vec, dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups);
+        else hipLaunchKernelGGL(one, dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups);
+    };
+    constexpr int V = 16 / (int)sizeof(VT);   // rows of a streamed layout's group
     if (part == RSTEP_P) {
-        const int grid = std::min((A->n + kResBS - 1) / kResBS, 2048);
+        const int grid = std::min((A->n + kResBS - 1) / kResBS, 1024);
         hipLaunchKernelGGL(k_cg_step_p<VT>, dim3(grid), dim3(kResBS), 0, s, a);
     } else if (part == RSTEP_ALPHA) {
-        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_ALPHA>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+        sums(k_cg_step<VT, RSTEP_ALPHA, 1>, k_cg_step<VT, RSTEP_ALPHA, V>);
     } else if (part == RSTEP_UPDATE) {
-        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_UPDATE>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+        sums(k_cg_step<VT, RSTEP_UPDATE, 1>, k_cg_step<VT, RSTEP_UPDATE, V>);
     } else {
         // a launch of one workgroup has not set the words
         hipLaunchKernelGGL(k_resident_begin, dim3((kSlotGens * kSlotGen + 255) / 256), dim3(256), 0, s, a.S, RS_OPEN);
-        hipLaunchKernelGGL((k_cg_step<VT, RSTEP_RESID>), dim3(plan.grid), dim3(kResBS), 0, s, a, q, groups, per);
+        sums(k_cg_step<VT, RSTEP_RESID, 1>, k_cg_step<VT, RSTEP_RESID, V>);
     }
     M4_HIP(hipGetLastError());
     return MTL4G_OK;
