@@ -505,6 +505,23 @@ int upload_sweep(const SweepRows& R, int fmt, Sweep* S) {
         lev_blk[l + 1] = lev_blk[l] + nb;
         for (int32_t i = 0; i < nb; i++) blk_level.push_back(l);
     }
+    // Entries requested before the wait.  A row with more costs its level another
+    // round trip (0.35 us per level with 4 entries instead of 8, 0.25 to 0.45 with 8
+    // instead of 16), requests past a row's end cost every level (0.08 us with 8, 0.3
+    // more with 16): 8 pays where a quarter of the levels has a row longer than 4,
+    // 16 where half of them has one longer than 8.  One solve(P, x) with 4 / 8 / 16:
+    // 5-point grid of 90,300 rows (rows of 2) 1140 / 1233 / 1575 us; 7-point grid of
+    // 125,000 rows in random order (up to 6, in 17 of 18 levels more than 4) 188 /
+    // 172 / 176; random graphs of 120,011 rows, mean length 2: 198 / 185 / 177, 5.5:
+    // 292 / 254 / 248.
+    int32_t over4 = 0, over8 = 0;
+    for (int32_t l = 0; l < nlev; l++) {
+        int32_t longest = 0;
+        for (int32_t k = lev_ptr[l]; k < lev_ptr[l + 1]; k++) longest = std::max(longest, rowptr[k + 1] - rowptr[k]);
+        over4 += longest > 4;
+        over8 += longest > 8;
+    }
+    S->ahead = 2 * over8 > nlev ? 16 : 4 * over4 > nlev ? 8 : 4;
     S->n = n;
     S->nnz = nnz;
     S->nlev = nlev;
@@ -716,15 +733,9 @@ static void launch_levels(const Sweep& S, const MT* val, const MT* dia, const IT
     const SweepView<MT, VT> V{S.perm.p, S.rowptr.p, S.col.p, S.lev_ptr.p, S.lev_blk.p,
                               S.blk_level.p, val, dia, S.nlev, S.unit ? 1 : 0};
     const dim3 grid(S.nblocks), block(kSweepBS);
-    // Entries requested before the wait: a row with more pays another round trip
-    // on its level's path, one with fewer issues the loads for nothing.  Two
-    // sweeps of a graph's factor (120,011 rows, 5.5 entries per row, up to 16 and
-    // more): 265 us with 4, 234 with 8, 222 with 16; of a 5-point factor
-    // (90,000 rows, 2 entries): 1129, 1226 and 1581 us.  The line between lies
-    // where a row of the mean length and a few more still fits.
-    if (S.nnz <= 3 * (int64_t)S.n)
+    if (S.ahead == 4)
         hipLaunchKernelGGL((k_sweep<kSweepBS, 4, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
-    else if (S.nnz <= 4 * (int64_t)S.n)
+    else if (S.ahead == 8)
         hipLaunchKernelGGL((k_sweep<kSweepBS, 8, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);
     else
         hipLaunchKernelGGL((k_sweep<kSweepBS, 16, MT, IT, VT>), grid, block, 0, s, V, v, w, w32, counters, err, skip);

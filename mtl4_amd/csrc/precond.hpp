@@ -26,6 +26,7 @@ struct ChainSweep;
 struct Sweep {
     int32_t n = 0, nlev = 0, nblocks = 0;
     int64_t nnz = 0;
+    int ahead = 16;              // entries of a row the level schedule requests before its wait: 4, 8 or 16
     bool unit = false;
     DevBuf<int32_t> perm, rowptr, col, lev_ptr, lev_blk, blk_level;
     DevBuf<int32_t> src, dsrc;   // values gathered from a device factor: entry / diagonal sources
