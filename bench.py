@@ -783,9 +783,12 @@ def main():
     torch.cuda.synchronize()
     t_fp64 = time.perf_counter() - t0
     iters = it.iterations()
-    # the roofline kernel inside the solve: one more solve with HIP events
-    # around each of its products (on the solve's stream)
     Lb = m._lib.lib()
+    chip = m._lib.CgChipInfo()   # how the timed solves ran (operand 0: launch per kernel)
+    m._lib.check(Lb.mtl4g_cg_chip(C.byref(chip)))
+    # the product q = A*p of that solve: one more solve with HIP events around
+    # each of its products (on the solve's stream).  An on-chip solve forms it
+    # inside its kernel; the product's own kernel then runs beside each iteration
     tot_us, cnt = C.c_double(), C.c_int64()
     m._lib.check(Lb.mtl4g_set_product_timing(1))
     m._lib.check(Lb.mtl4g_product_timing(C.byref(tot_us), C.byref(cnt)))
@@ -799,15 +802,18 @@ def main():
                                              "avg_launch_us")}
         cold["note"] = ("the same product with y = A*x alone, each launch after 14 vector passes of torch "
                         "kernels (459 MB) that leave little of the matrix in the MALL")
-        # the PMC record of the in-solve product holds for the configuration it was taken on
+        # the PMC record of the in-solve product holds for the configuration it was
+        # taken on, and for the product fused with p.q of a launch-per-kernel solve
         try:
             rec = json.load(open(os.path.join(ROOT, "profiles", "spmv_diffusion3d_160_traffic.json")))
             rec = rec["configs"]["cg_product_in_solve"]
-            q_traffic = rec["traffic_bytes"] if rec.get("config") == traffic_key(m, kern, grid) else None
+            q_traffic = rec["traffic_bytes"] if not chip.operand and rec.get("config") == traffic_key(m, kern, grid) else None
         except (OSError, ValueError, KeyError):
             q_traffic = None
         roofline.update({
-            "kernel": "%s<EpiCgQ> (q = A*p fused with p.q inside the timed FP64 CG solve, diffusion3d %d^3)"
+            "kernel": ("%s<EpiCgProduct> (q = A*p launched beside each iteration of an on-chip FP64 CG solve, "
+                       "which forms it inside its own kernel; diffusion3d %d^3)" if chip.operand else
+                       "%s<EpiCgQ> (q = A*p fused with p.q inside the timed FP64 CG solve, diffusion3d %d^3)")
                       % (kname, g),
             "timing": ("HIP events around each of the %d products of one FP64 CG solve, on the solve's "
                        "stream (mtl4g_set_product_timing)" % cnt.value),
@@ -819,6 +825,32 @@ def main():
                                "note": "the CSR bytes of y = A*x over the same time"},
             "avg_launch_us": round(q_us, 2),
             "cold_mall_context": cold})
+    chip_bytes = None
+    if chip.operand == 6:
+        # the kernel of the timed solves: per iteration its stored matrix values,
+        # p at the diagonals beyond the LDS halo, p written once and, where a lane
+        # has more than 16 rows, the inverse diagonal and x twice
+        far = 2 if g * g > 1024 else 0
+        chip_bytes = by_layout - 16 * n + 8 * n * (far + 1 + (3 if chip.rows_per_lane > 16 else 0))
+        it_us = 1e6 * t_fp64 / args.steps / max(iters, 1)
+        key = "%s/%d" % (layout, chip.rows_per_lane)
+        try:
+            rec = json.load(open(os.path.join(ROOT, "profiles", "cg_on_chip_traffic.json")))["configs"].get(key)
+            chip_traffic = rec["traffic_bytes_per_iteration"] if rec and rec["N"] == n else None
+        except (OSError, ValueError, KeyError):
+            chip_traffic = None
+        roofline = {"bound": "hbm",
+                    "kernel": "k_cg_large (itl::cg + pc::diagonal, FP64, whole iterations on the chip, %d per launch, "
+                              "%s layout streamed, %d rows per lane; diffusion3d %d^3)"
+                              % (chip.steps, layout, chip.rows_per_lane, g),
+                    "config": key, "workgroups": chip.workgroups,
+                    "timing": "wall time of the timed solves by their iterations",
+                    "achieved": round(chip_bytes / it_us / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(chip_bytes / it_us / 1e3 / HBM_PEAK_GBS, 4), "traffic": chip_traffic,
+                    "layout": layout, "bytes_per_iteration": chip_bytes, "us_per_iteration": round(it_us, 2),
+                    "note": "bytes the iteration cannot do without; traffic: bytes past the L2 per iteration "
+                            "(rocprofv3), with the registers that are kept in scratch",
+                    "hbm_context": roofline.pop("hbm_context"), "product": roofline}
     r = m.dense_vector(n)
     r.assign(b)
     A.mult(x, r, m.MINUS)
@@ -890,7 +922,7 @@ def main():
                                                            big_rows=args.serve_big_rows))
 
     v = args.steps / t_fp64
-    it_bytes = by_layout + 11 * 8 * n
+    it_bytes = chip_bytes or by_layout + 11 * 8 * n
     mixed["speedup_vs_fp64"] = round(mixed["solves_per_s"] / v, 3)
     mixed_bf16["speedup_vs_fp64"] = round(mixed_bf16["solves_per_s"] / v, 3)
     mixed["recurrence"] = "cg + diagonal in FP32 on FP32 values, FP64 residual refresh at 0.1x"
@@ -918,10 +950,11 @@ def main():
         "p99_ms": round(1000 * float(np.percentile(lat, 99)), 3),
         "mixed": mixed,
         "mixed_bf16": mixed_bf16,
-        "cg_iteration": {"us": round(1e6 * t_fp64 / args.steps / max(iters, 1), 2),
+        "cg_iteration": {"operand": chip.operand, "us": round(1e6 * t_fp64 / args.steps / max(iters, 1), 2),
                          "bytes": it_bytes, "GBs": round(it_bytes * iters * args.steps / t_fp64 / 1e9, 1),
                          "frac": round(it_bytes * iters * args.steps / t_fp64 / 1e9 / HBM_PEAK_GBS, 4),
-                         "note": "the layout's SpMV bytes + 11 vector passes (P: 4, XR: 7): the bytes of the "
+                         "note": "the bytes of roofline.bytes_per_iteration" if chip_bytes else
+                                 "the layout's SpMV bytes + 11 vector passes (P: 4, XR: 7): the bytes of the "
                                  "launch-per-kernel loop; a solve kept on the chip moves fewer"},
         "spmv": {"diffusion3d_f64_GBs": round(ctx_gbs, 1), "diffusion3d_f64_back_to_back_GBs": round(spmv_gbs, 1),
                  "random_2M_poisson16_f64_GBs": round(rnd_gbs, 1),

@@ -12,17 +12,18 @@
 // or store stands in the computing wave's way.  Inside a tile the chains cx-1
 // and cy-1 hand over their element of the previous step lane to lane (DPP,
 // ds_bpermute), between tiles through memory (the tile's last chains' rows in
-// exchange slots, polled while they are empty).  The waves meet at one barrier per block of U steps.
+// exchange slots, polled while they are empty).  The waves meet at one barrier
+// per block of U steps.
 //
 // Memory access is coalesced although the chains' rows lie Lc apart: the
 // factor's values are stored tile by tile in step-major order (slot =
 // tile*stile + (step - first step of the tile)*64 + lane), so a block's values
 // are contiguous and go to LDS directly, three blocks ahead; the input and
 // output vectors keep their natural order and move through LDS in blocks of U
-// steps (8 consecutive rows of a chain per 8 lanes).  Every row is computed by one lane with MTL4's
-// subtraction order (ascending columns, lower_trisolve.hpp:174-209,
-// upper_trisolve.hpp:161-176), so the results are the level-scheduled
-// sweep's bit for bit.
+// steps (8 consecutive rows of a chain per 8 lanes).  Every row is computed by
+// one lane with MTL4's subtraction order (ascending columns,
+// lower_trisolve.hpp:174-209, upper_trisolve.hpp:161-176), so the results are
+// the level-scheduled sweep's bit for bit.
 #pragma once
 
 #include <vector>

@@ -66,7 +66,7 @@ __device__ __forceinline__ VT res_ld(const VT* p, int i) {
 template <typename VT, int ND_, int R_>
 struct OpDia {
     static constexpr int R = R_, ND = ND_, kRegs = R_ * ND_;
-    static constexpr bool kOne = true;   // runs as one workgroup without p in memory
+    static constexpr bool kOne = R_ <= 8;   // runs as one workgroup (up to 4096 rows) without p in memory
     static constexpr int LDS = R * kResBS + 2 * kResHalo;
     VT v[R][ND];
     unsigned mask[R];

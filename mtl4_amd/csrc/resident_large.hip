@@ -1,12 +1,19 @@
 // resident_large.hip -- itl::cg + pc::identity / pc::diagonal (cg.hpp:38-111) on
 // diagonal layouts whose values no longer fit the registers (resident.hip): the
-// matrix is streamed; r and q stay in registers, the workgroup's p in LDS, and up
-// to kLargeKeep groups per lane also x and the inverse diagonal in registers.
+// matrix is streamed; r and q are a lane's own (registers, and scratch where these
+// run out), the workgroup's p is in LDS, and up to kLargeKeep groups per lane x and
+// the inverse diagonal are kept as r is.
 //
-// What bounds it: memory.  Per iteration a row of the FP64 symmetric layout moves
+// What bounds it: memory.  Per iteration a row of the FP64 symmetric layout needs
 // its 4 stored values, the far neighbours' p (2, at agent scope, past the L2), one
 // write of p and, if they are streamed, the inverse diagonal and x twice: 80 bytes
 // where the three-launch loop moves 136; 56 with x and the inverse diagonal kept.
+// Moved past the L2 (counters): 441 MB per iteration at 160^3 where 328 are needed,
+// 137 at 126^3 for 112.  The difference is scratch: with 16 groups r and q are 128
+// of the 256 registers and the rest does not hold what a group in work needs, so
+// the compiler stores and reloads part of r every iteration (7 diagonals: 396 bytes
+// per lane at 16 groups, 256 at 14, 64 at 10, none at 9, 128 at 8 with x and the
+// inverse diagonal kept).
 // On top come one exchange of p and two all-reduces, about 9 us.  Measured per
 // iteration, FP64, diagonal preconditioner, three launches -> here (symmetric
 // layout; plain one in parentheses): 102^3 42.0 -> 15.5 us (47.8 -> 17.6), 126^3
@@ -39,8 +46,10 @@ struct ResVec<float> {
 };
 constexpr int kResSc1 = 16;   // buffer cache policy: agent scope, as ld_agent / st_agent
 constexpr int kResNt = 2;     // non-temporal: streamed once per iteration
-// Groups per lane up to which x and the inverse diagonal stay in registers: four
-// arrays of 16 bytes per group, 128 of a lane's 256 registers.
+// Groups per lane up to which x and the inverse diagonal are kept: four arrays of 16
+// bytes per group, 128 of a lane's 256 registers.  At 8 groups (126^3) 30.4 us per
+// iteration against 33 with both streamed, although 128 bytes per lane go to scratch;
+// more groups kept were not measured.
 constexpr int kLargeKeep = 8;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t res_rsrc(const void* p, int bytes) {
