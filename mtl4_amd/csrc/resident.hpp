@@ -96,6 +96,9 @@ int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
         M4_HIP(hipStreamSynchronize(s));
         return MTL4G_OK;
     };
+    // work that the caller has queued before the solve ends first: units that wait
+    // for it would keep other solves from an idle GPU
+    if (W.queued && plan.grid > 1) M4_HIP(hipStreamSynchronize(s));
     int launches = 1, chunk = kStepsMin;
     for (;;) {
         {

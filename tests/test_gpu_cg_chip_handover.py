@@ -217,3 +217,70 @@ def test_a_waiting_solve_is_served_in_turn(m):
     assert not any(t.is_alive() for t in ts)
     print("short ended %.0f ms before long" % (1e3 * (done["long"] - done["short"])), flush=True)
     assert done["short"] < done["long"]
+
+
+def test_a_solve_behind_queued_work_keeps_nobody_waiting(m):
+    """A solve on a stream with other work under way takes no compute units until
+    that has ended: a solve on an idle stream ends first."""
+    import torch
+    rp, ci, va = _matrix("grid3d", (61, 61, 61))
+    n = len(rp) - 1
+    A = m.compressed2D(n, n, rp, ci, va)
+    b = m.dense_vector(np.random.default_rng(5).uniform(-1, 1, n))
+    want, hist, _ = _cg(m, A, None, b, 50)
+    y = torch.zeros(64, device="cuda")
+    solvers = {k: m.Solver(A) for k in ("queued", "idle")}   # no allocation, which waits for the device, in the solves
+    for S in solvers.values():
+        S.solve(m.dense_vector(n), b, m.basic_iteration(1.0, 2, 0.0))
+
+    def timed(f):
+        torch.cuda.synchronize()
+        t0 = time.time()
+        f()
+        return time.time() - t0
+
+    def nap(count, s):   # kernels of one workgroup that end by the clock
+        with torch.cuda.stream(s):
+            for _ in range(count):
+                torch.cuda._sleep(10 ** 6)
+
+    def add(s):
+        with torch.cuda.stream(s):
+            y.add_(1)
+        s.synchronize()
+
+    queued = torch.cuda.Stream()
+    nap(1, queued)
+    each = timed(lambda: (nap(10, queued), queued.synchronize())) / 10
+    naps = max(1, min(2000, int(0.4 / each)))
+    # a stream that does not share the other's hardware queue
+    idle = None
+    for s in [torch.cuda.Stream() for _ in range(8)]:
+        add(s)
+        if timed(lambda: (nap(naps, queued), add(s))) < 0.2:
+            idle = s
+            break
+    torch.cuda.synchronize()
+    assert idle is not None
+    ended, xs = {}, {}
+
+    def work(name, s, delay, count):
+        with torch.cuda.stream(s):
+            time.sleep(delay)
+            x = m.dense_vector(n)
+            s.synchronize()
+            nap(count, s)
+            solvers[name].solve(x, b, m.basic_iteration(1.0, 50, 0.0))
+            ended[name], xs[name] = time.time(), x.numpy()
+
+    ts = [threading.Thread(target=work, args=a)
+          for a in (("queued", queued, 0, naps), ("idle", idle, 0.1, 0))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    assert not any(t.is_alive() for t in ts)
+    print("%d naps of %.2f ms; idle ended %.0f ms before queued"
+          % (naps, 1e3 * each, 1e3 * (ended["queued"] - ended["idle"])), flush=True)
+    assert ended["idle"] < ended["queued"]
+    assert np.array_equal(xs["idle"], want) and np.array_equal(xs["queued"], want)
