@@ -1701,13 +1701,6 @@ static int ensure_workspace(Workspace<VT>& W, int32_t n, int nvec, const mtl4g_p
     return MTL4G_OK;
 }
 
-// whether work is under way on s (Workspace::queued)
-static bool stream_busy(hipStream_t s) {
-    const bool busy = hipStreamQuery(s) == hipErrorNotReady;
-    if (busy) (void)hipGetLastError();   // not an error of the next launch
-    return busy;
-}
-
 // Events around the products of CG iterations (mtl4g_set_product_timing);
 // created on first use and kept for the process.
 struct ProductTimer {
@@ -1950,7 +1943,6 @@ int krylov_run(const mtl4g_matrix_s* A, const mtl4g_pc_s* P, int method, int fmt
     }
     const int nvec = method == MTL4G_CG ? 5 : 9;
     g_timer.used = 0;   // events of a solve that ended in an error are not counted
-    if (method == MTL4G_CG) W.queued = stream_busy(s);
     M4_TRY(ensure_workspace(W, A->n, nvec, P, hist_cap, s));
     Ctl init;
     std::memset(&init, 0, sizeof init);
@@ -2641,7 +2633,6 @@ int mixed_run(mtl4g_matrix_s* A, const mtl4g_pc_s* P, int method, int fmt, doubl
         return 0;
     }
     const bool bicg = method == MTL4G_BICGSTAB;
-    W.queued = stream_busy(s);
     if (bicg) M4_TRY(ensure_workspace(W64, A->n, 9, P, 0, s));
     else M4_TRY(ensure_workspace(W, A->n, 5, P, 0, s));
     Ctl* ctl = bicg ? W64.ctl.p : W.ctl.p;

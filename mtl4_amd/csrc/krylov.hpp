@@ -41,7 +41,6 @@ struct Workspace {
     DevBuf<double> pc64;      // float vectors with ilu_0/ic_0: the sweeps' FP64 chains (2n)
     DevBuf<double> rslots;    // resident CG: all-reduce slots and wait words (resident.hip)
     DevBuf<unsigned> rwords;
-    bool queued = false;      // the caller's stream had other work under way when the solve was called
     bool shared_gpu = false;  // other solves run beside this one: no grid that must hold the whole GPU
     Ctl* h_ctl = nullptr;     // pinned mirror for polling
     ~Workspace() {

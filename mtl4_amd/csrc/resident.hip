@@ -29,8 +29,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
-#include <map>
 #include <mutex>
 
 #include "resident_dev.hpp"
@@ -503,12 +503,13 @@ __global__ __launch_bounds__(kResBS) void k_cg_step(ResArgs a, const VT* q, int 
 namespace {
 struct Units {
     struct Device {
-        int used = 0;                        // CUs held by resident grids
-        uint64_t arrived = 0, served = 0;    // claims, in order
+        int used = 0;                     // CUs held by resident grids
+        ResidentClaim* first = nullptr;   // claims that wait, in the order of arrival
     };
     std::mutex mu;
     std::condition_variable cv;
-    std::map<int, Device> devices;
+    Device devices[64];
+    Device& of(int device) { return devices[(unsigned)device % 64]; }
 };
 Units& units() {
     static Units u;
@@ -516,15 +517,22 @@ Units& units() {
 }
 }  // namespace
 
-ResidentClaim::ResidentClaim(int dev, int n, int total) : device(dev), units(std::min(n, total)) {
+ResidentClaim::ResidentClaim(int dev, int n, int total, int wait_ms)
+    : device(dev), units(std::min(n, total)), wanted(n > 0) {
     if (!units) return;
     Units& u = mtl4g::units();
     std::unique_lock<std::mutex> lk(u.mu);
-    Units::Device& d = u.devices[device];
-    const uint64_t turn = d.arrived++;
-    u.cv.wait(lk, [&] { return d.served == turn && d.used + units <= total; });
-    d.used += units;
-    d.served++;
+    Units::Device& d = u.of(device);
+    int ahead = 1;   // the holder
+    ResidentClaim** at = &d.first;
+    for (; *at; at = &(*at)->next) ahead++;
+    *at = this;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(wait_ms) * ahead;
+    const bool mine = u.cv.wait_until(lk, until, [&] { return d.first == this && d.used + units <= total; });
+    for (at = &d.first; *at != this; at = &(*at)->next) {}
+    *at = next;
+    if (mine) d.used += units;
+    else units = 0;
     lk.unlock();
     u.cv.notify_all();
 }
@@ -534,7 +542,7 @@ ResidentClaim::~ResidentClaim() {
     Units& u = mtl4g::units();
     {
         std::lock_guard<std::mutex> lk(u.mu);
-        u.devices[device].used -= units;
+        u.of(device).used -= units;
     }
     u.cv.notify_all();
 }

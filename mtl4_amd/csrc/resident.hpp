@@ -54,14 +54,22 @@ mtl4g_cg_chip_info& resident_info();
 // that spans several workgroups takes its CUs before it is launched and gives
 // them back after it has finished, so two such grids never wait for each
 // other's CUs.  Served in the order of arrival: a solve that gives its units
-// back and asks again at once stands behind those that waited.
+// back and asks again at once stands behind those that waited.  A claim waits at
+// most wait_ms per claim before it and then stands for nothing (held() false):
+// whoever holds the units may itself be waiting, for earlier work on its stream.
+// The caller launches all the same; two grids that meet are refused and go on in
+// single steps.
 struct ResidentClaim {
     int device, units;
-    ResidentClaim(int device, int units, int total);
+    bool wanted;
+    ResidentClaim* next = nullptr;   // behind this one in the queue
+    ResidentClaim(int device, int units, int total, int wait_ms);
     ~ResidentClaim();
+    bool held() const { return units > 0 || !wanted; }
     ResidentClaim(const ResidentClaim&) = delete;
     ResidentClaim& operator=(const ResidentClaim&) = delete;
 };
+constexpr int kClaimWait = 30;   // a holder's launches take about 20 ms at most (four of 5 ms)
 
 // Iterations per launch, so that other streams' kernels wait no more than about
 // 5 ms for the compute units: 256 of up to 20 us while the matrix is in
@@ -96,13 +104,11 @@ int resident_cg(const mtl4g_matrix_s* A, int value_format, const void* inv_diag,
         M4_HIP(hipStreamSynchronize(s));
         return MTL4G_OK;
     };
-    // work that the caller has queued before the solve ends first: units that wait
-    // for it would keep other solves from an idle GPU
-    if (W.queued && plan.grid > 1) M4_HIP(hipStreamSynchronize(s));
-    int launches = 1, chunk = kStepsMin;
+    int launches = 1, chunk = kStepsMin, wait = kClaimWait;
     for (;;) {
         {
-            ResidentClaim claim(A->device, plan.grid > 1 ? plan.grid : 0, A->cus);
+            ResidentClaim claim(A->device, plan.grid > 1 ? plan.grid : 0, A->cus, wait);
+            wait = claim.held() ? kClaimWait : 0;   // waited once: from then on only where units are free
             for (int k = 0; k < launches; k++) {
                 M4_TRY(resident_launch<VT>(plan, A, value_format, inv_diag, dfmt, W, x, steps, s));
                 M4_TRY(after());

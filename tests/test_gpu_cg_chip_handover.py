@@ -220,8 +220,9 @@ def test_a_waiting_solve_is_served_in_turn(m):
 
 
 def test_a_solve_behind_queued_work_keeps_nobody_waiting(m):
-    """A solve on a stream with other work under way takes no compute units until
-    that has ended: a solve on an idle stream ends first."""
+    """A solve on a stream with other work under way has claimed compute units that it
+    does not use yet: a solve on an idle stream waits for them for a while at most, and
+    ends first."""
     import torch
     rp, ci, va = _matrix("grid3d", (61, 61, 61))
     n = len(rp) - 1
